@@ -86,9 +86,39 @@ template <int DT, int HD, int GPW> const void* decode_kernel() {
     return reinterpret_cast<const void*>(&paged_decode_stream_kernel<DT, HD, GPW>);
 }
 
-// Up to this many (sequence, head) pairs the combine gives each pair two waves (at most
-// 4,096 waves: all resident on a 256-CU part); larger batches get one wave per pair.
-constexpr int kCombineSplitPairs = PKV_DECODE_COMBINE_SPLIT_PAIRS;
+// Waves the combine gives each (sequence, head) pair: there are as many ranges for any
+// batch, so with few pairs each has many records, and one wave folds them in dependent
+// trips of a few rows each. Whole decode calls with 1 / 2 / 4 / 8 / 16 waves per pair (us):
+//   32 pairs (1 sequence of 20,011 tokens, hd 128)  45.2 / 34.8 / 28.7 / 26.2 / 25.7
+//   64 pairs (2 sequences of 3,000-9,000)           33.7 / 26.8 / 21.9 / 20.6 / 20.5
+//   128 pairs (4 such)                              32.8 / 29.3 / 27.1 / 26.2 / 26.8
+//   256 pairs (8 such)                              42.6 / 41.1 / 39.6 / 39.8 / 40.3
+//   512 pairs (16 of 1,000-4,000)                   35.0 / 34.2 / 34.1 / 34.4 / 38.0
+//   1,024 pairs (64 of 200-3,000, 16 heads)         71.3 / 71.4 / 72.1 / 74.6 / 77.9
+//   1,024 pairs (32 of 128-32,768, log)            106.9 / 105.7 / 105.0 / 106.5 / 110.1
+//   1,536 pairs (64 of 1,024-4,096, 24 heads)      109.8 / 110.0 / 111.6 / 115.0 / 119.8
+int combine_waves(int pairs) {
+  if (pairs <= 64) return 16;
+  if (pairs <= 256) return 8;
+  if (pairs <= 512) return 4;
+  return pairs <= PKV_DECODE_COMBINE_SPLIT_PAIRS ? 2 : 1;
+}
+template <int DT, int HD, int SP, bool WT>
+void launch_combine_sp(const DecodeArgs& a, hipStream_t st) {
+  constexpr int WG = SP > 4 ? SP : 4;  // waves per workgroup
+  const int pairs = a.batch * a.nh;
+  hipLaunchKernelGGL((paged_decode_combine_kernel<DT, HD, SP, WT>),
+                     dim3((unsigned)((pairs + WG / SP - 1) / (WG / SP))), dim3(kWave * WG), 0, st, a);
+}
+template <int DT, int HD, bool WT> void launch_combine(const DecodeArgs& a, hipStream_t st) {
+  switch (combine_waves(a.batch * a.nh)) {
+    case 16: return launch_combine_sp<DT, HD, 16, WT>(a, st);
+    case 8: return launch_combine_sp<DT, HD, 8, WT>(a, st);
+    case 4: return launch_combine_sp<DT, HD, 4, WT>(a, st);
+    case 2: return launch_combine_sp<DT, HD, 2, WT>(a, st);
+    default: return launch_combine_sp<DT, HD, 1, WT>(a, st);
+  }
+}
 
 struct LaunchDecode {
   const DecodeArgs* a;
@@ -116,16 +146,13 @@ struct LaunchDecode {
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || (a->num_wg <= 1 && !a->pre_row)) return e;
-    const int pairs = a->batch * a->nh;  // (sequence, query head) pairs
-    const dim3 g2((unsigned)((pairs + 1) / 2)), g1((unsigned)((pairs + 3) / 4));
-    if (one && pairs <= kCombineSplitPairs)  // after a one-launch cascade: its unit split
-      hipLaunchKernelGGL((paged_decode_combine_kernel<DT, HD, 2, true>), g2, dim3(256), 0, st, *a);
-    else if (one)
-      hipLaunchKernelGGL((paged_decode_combine_kernel<DT, HD, 1, true>), g1, dim3(256), 0, st, *a);
-    else if (pairs <= kCombineSplitPairs)
-      hipLaunchKernelGGL((paged_decode_combine_kernel<DT, HD, 2>), g2, dim3(256), 0, st, *a);
-    else
-      hipLaunchKernelGGL((paged_decode_combine_kernel<DT, HD, 1>), g1, dim3(256), 0, st, *a);
+    if constexpr (use_mfma<DT, HD>()) {
+      if (one) {  // after a one-launch cascade: its unit split
+        launch_combine<DT, HD, true>(*a, st);
+        return hipGetLastError();
+      }
+    }
+    launch_combine<DT, HD, false>(*a, st);
     return hipGetLastError();
   }
 };
