@@ -133,7 +133,7 @@ int64_t pkv_decode_workspace_bytes(int32_t num_workgroups, int32_t batch, int32_
  * for every context length): small batches of 16-bit K/V at head_dim 64 or 128 whose
  * (sequence, KV head) pairs fit the CUs and whose table width is at most 2,048 tokens
  * run one kernel with one workgroup per (sequence, KV head, sub-group of its query
- * heads -- as few heads as keep the workgroups within the CUs) that splits the
+ * heads -- as few heads, 16 at most, as keep the workgroups within the CUs) that splits the
  * sequence among its waves and merges in LDS (no workspace used); everything else the
  * split above with pkv_decode_workgroups() workgroups, whose workspace size the caller
  * passes.

@@ -35,18 +35,24 @@ template <int DT, int GPW, int HD>
 __global__ void __launch_bounds__(512)
 cascade_decode_kernel(const DecodeArgs d, const PrefillArgs p, const int prefix_wg,
                       const int items) {
+  // The prefix items' K/V rings; the stream pass's waves stage V rows in the same memory
+  // (a prefix workgroup's items end with a barrier before it streams).
+  __shared__ __align__(16) PrefillLds<HD> lds;
+  static_assert(sizeof(lds) >= PKV_DECODE_WAVES_PER_WG * kVSlotBytes, "V slots fit the rings");
+  u32x4* const vslots = &lds.ring[0][0][0][0];
   const int bx = (int)blockIdx.x;
   if (bx < prefix_wg) {
     const int workers = prefix_wg * (int)gridDim.y;
     for (int it = (int)blockIdx.y * prefix_wg + bx; it < items; it += workers) {
-      prefill_item<DT, HD, true>(p, it);
+      prefill_item<DT, HD, true>(p, it, lds);
       __syncthreads();  // the item's merge used the rings the next item's loads fill
     }
     if (d.num_wg == d.full_wg) return;  // no stream share for prefix workgroups
-    decode_mfma_body<DT, GPW, true, HD, false, true, true>(d, d.full_wg + bx, (int)blockIdx.y);
+    decode_mfma_body<DT, GPW, true, HD, false, true, true>(d, d.full_wg + bx, (int)blockIdx.y,
+                                                             vslots);
     return;
   }
-  decode_mfma_body<DT, GPW, true, HD, false, true, true>(d, bx - prefix_wg, (int)blockIdx.y);
+  decode_mfma_body<DT, GPW, true, HD, false, true, true>(d, bx - prefix_wg, (int)blockIdx.y, vslots);
 }
 
 template <int DT, int HD>
@@ -71,8 +77,12 @@ hipError_t launch_hd(const DecodeArgs& d, PrefillArgs p, int64_t rows, int gpw, 
     case 3:
       hipLaunchKernelGGL((cascade_decode_kernel<DT, 3, HD>), grid, block, 0, st, d, p, prefix_wg, n);
       break;
-    default:
+    case 4:
       hipLaunchKernelGGL((cascade_decode_kernel<DT, 4, HD>), grid, block, 0, st, d, p, prefix_wg, n);
+      break;
+    default:
+      hipLaunchKernelGGL((cascade_decode_kernel<DT, kWideHeads, HD>), grid, block, 0, st, d, p,
+                         prefix_wg, n);
       break;
   }
   return hipGetLastError();
@@ -91,7 +101,7 @@ bool cascade_one_launch_shape(int kv_dtype, int head_dim, int block_size, int ba
 
 hipError_t launch_cascade(const DecodeArgs& d, const PrefillArgs& p, int64_t rows, int kv_dtype,
                           int head_dim, int gpw, int prefix_wg, int ygrid, hipStream_t st) {
-  if (!cascade_one_launch_shape(kv_dtype, head_dim, d.bs, d.batch, 8) || gpw < 1 || gpw > 4 ||
+  if (!cascade_one_launch_shape(kv_dtype, head_dim, d.bs, d.batch, 8) || gpw < 1 || gpw > kWideHeads ||
       p.bs_shift < 0)
     return hipErrorInvalidValue;
   if (kv_dtype == PKV_BF16)

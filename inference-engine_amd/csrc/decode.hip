@@ -48,13 +48,22 @@ DecodeWs decode_ws(int32_t num_wg, int32_t batch, int32_t nh, int32_t hd, bool c
   return w;
 }
 
+// The MFMA kernel serves 16-bit K/V at head_dim 64 and 128; every other shape uses the
+// generic stream kernel.
+template <int DT, int HD> constexpr bool use_mfma() {
+  return DT != PKV_F32 && (HD == 128 || HD == 64) && PKV_DECODE_USE_MFMA;
+}
+
 // Run f.run<DT, HD, GPW>() for the runtime (dtype, head_dim, heads per wave).
 template <int DT, int HD, class F> hipError_t by_gpw(int gpw, const F& f) {
   switch (gpw) {
     case 1: return f.template run<DT, HD, 1>();
     case 2: return f.template run<DT, HD, 2>();
     case 3: return f.template run<DT, HD, 3>();
-    default: return f.template run<DT, HD, 4>();
+    case 4: return f.template run<DT, HD, 4>();
+    default:  // only planned where the MFMA kernel serves the shape (plan_decode)
+      if constexpr (use_mfma<DT, HD>()) return f.template run<DT, HD, kWideHeads>();
+      else return hipErrorInvalidValue;
   }
 }
 template <int DT, class F> hipError_t by_hd(int hd, int gpw, const F& f) {
@@ -74,16 +83,16 @@ template <class F> hipError_t by_dtype(int dt, int hd, int gpw, const F& f) {
   }
 }
 
-// The MFMA kernel serves 16-bit K/V at head_dim 128; every other shape uses the
-// generic stream kernel.
-template <int DT, int HD> constexpr bool use_mfma() {
-  return DT != PKV_F32 && (HD == 128 || HD == 64) && PKV_DECODE_USE_MFMA;
-}
 template <int DT, int HD, int GPW> const void* decode_kernel() {
   if constexpr (use_mfma<DT, HD>())
     return reinterpret_cast<const void*>(&paged_decode_mfma_kernel<DT, GPW, true, HD, false>);
   else
     return reinterpret_cast<const void*>(&paged_decode_stream_kernel<DT, HD, GPW>);
+}
+
+// Dynamic LDS of the stream pass's workgroups of wpg waves.
+template <int DT, int HD, int GPW> constexpr unsigned stream_lds(int wpg) {
+  return use_mfma<DT, HD>() && pv_mfma<HD, GPW>() ? (unsigned)(wpg * kVSlotBytes) : 0u;
 }
 
 // Waves the combine gives each (sequence, head) pair: there are as many ranges for any
@@ -127,20 +136,21 @@ struct LaunchDecode {
   const CascadeLaunch* one = nullptr;  // non-null: the stream pass shares a launch with a prefix pass
   template <int DT, int HD, int GPW> hipError_t run() const {
     const dim3 grid((unsigned)a->num_wg, (unsigned)ygrid), block(kWave * wpg);
+    const unsigned lds = stream_lds<DT, HD, GPW>(wpg);
     if constexpr (use_mfma<DT, HD>()) {
       const bool staged = a->batch > kWave && a->batch <= kLdsBatch;
       if (one) {
-        const hipError_t e = launch_cascade(*a, *one->p, one->rows, DT, HD, GPW, one->prefix_wg,
+        const hipError_t e = launch_cascade(*a, *one->p, one->rows, DT, HD, a->gpw, one->prefix_wg,
                                             ygrid, st);
         if (e != hipSuccess) return e;
       } else if (a->bs % 16 == 0 && staged)
-        hipLaunchKernelGGL((paged_decode_mfma_kernel<DT, GPW, true, HD, false, true>), grid, block, 0, st, *a);
+        hipLaunchKernelGGL((paged_decode_mfma_kernel<DT, GPW, true, HD, false, true>), grid, block, lds, st, *a);
       else if (a->bs % 16 == 0)
-        hipLaunchKernelGGL((paged_decode_mfma_kernel<DT, GPW, true, HD, false>), grid, block, 0, st, *a);
+        hipLaunchKernelGGL((paged_decode_mfma_kernel<DT, GPW, true, HD, false>), grid, block, lds, st, *a);
       else if (staged)
-        hipLaunchKernelGGL((paged_decode_mfma_kernel<DT, GPW, false, HD, false, true>), grid, block, 0, st, *a);
+        hipLaunchKernelGGL((paged_decode_mfma_kernel<DT, GPW, false, HD, false, true>), grid, block, lds, st, *a);
       else
-        hipLaunchKernelGGL((paged_decode_mfma_kernel<DT, GPW, false, HD, false>), grid, block, 0, st, *a);
+        hipLaunchKernelGGL((paged_decode_mfma_kernel<DT, GPW, false, HD, false>), grid, block, lds, st, *a);
     } else {
       hipLaunchKernelGGL((paged_decode_stream_kernel<DT, HD, GPW>), grid, block, 0, st, *a);
     }
@@ -165,10 +175,11 @@ struct LaunchSplit {
   template <int DT, int HD, int GPW> hipError_t run() const {
     if constexpr (use_mfma<DT, HD>()) {
       const dim3 grid((unsigned)a->batch, (unsigned)ytasks), block(kWave * kSplitWaves);
+      const unsigned lds = pv_mfma<HD, GPW, true>() ? kSplitWaves * kVSlotBytes : 0;
       if (a->bs % 16 == 0)
-        hipLaunchKernelGGL((paged_decode_mfma_kernel<DT, GPW, true, HD, true>), grid, block, 0, st, *a);
+        hipLaunchKernelGGL((paged_decode_mfma_kernel<DT, GPW, true, HD, true>), grid, block, lds, st, *a);
       else
-        hipLaunchKernelGGL((paged_decode_mfma_kernel<DT, GPW, false, HD, true>), grid, block, 0, st, *a);
+        hipLaunchKernelGGL((paged_decode_mfma_kernel<DT, GPW, false, HD, true>), grid, block, lds, st, *a);
       return hipGetLastError();
     } else {
       return hipErrorInvalidValue;  // never chosen for these shapes
@@ -188,17 +199,22 @@ struct QueryDecode {
     *tile = DecodeShape<DT, HD>::TILE;
     if (!per_cu) return hipSuccess;
     return hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, decode_kernel<DT, HD, GPW>(),
-                                                         kWave * wpg, 0);
+                                                         kWave * wpg, stream_lds<DT, HD, GPW>(wpg));
   }
 };
 
 // Query heads per wave: the whole group when it has at most 4 heads (the register
-// budget of 4 heads x 8 fp32 accumulators keeps the kernel spill-free at hd 256), else
-// the largest of {4, 3, 2} that divides the group, else 1. Waves that share a KV head
-// read the same rows within a few hundred cycles of each other, so the repeat is served
-// from L2, not HBM.
-int pick_gpw(int groups) {
+// budget of 4 heads x 8 fp32 accumulators keeps the kernel spill-free at hd 256). Larger
+// groups: on the MFMA kernel (wide) the largest divisor of the group up to kWideHeads, whose
+// cost does not grow with the heads; else the largest of {4, 3, 2} that divides the group,
+// else 1, whose waves read the same rows within a few hundred cycles of each other, so the
+// repeat is served from L2, not HBM -- but through L2 once per wave.
+int pick_gpw(int groups, bool wide) {
   if (groups <= 4) return groups;
+  if (wide) {
+    for (int c = groups < kWideHeads ? groups : kWideHeads; c > 4; --c)
+      if (groups % c == 0) return c;
+  }
   const int cands[3] = {4, 3, 2};
   for (int c : cands)
     if (groups % c == 0) return c;
@@ -209,15 +225,39 @@ int pick_gpw(int groups) {
 struct DecodePlan {
   int gpw, nsub, wpg, ygrid;
 };
-DecodePlan plan_decode(int num_heads, int num_kv_heads) {
+DecodePlan plan_tasks(int num_heads, int num_kv_heads, bool wide) {
   DecodePlan p;
   const int groups = num_heads / num_kv_heads;
-  p.gpw = pick_gpw(groups);
+  p.gpw = pick_gpw(groups, wide);
   p.nsub = groups / p.gpw;
   const int tasks = num_kv_heads * p.nsub;
   p.wpg = tasks < PKV_DECODE_WAVES_PER_WG ? tasks : PKV_DECODE_WAVES_PER_WG;
   p.ygrid = (tasks + p.wpg - 1) / p.wpg;
   return p;
+}
+DecodePlan plan_decode(int kv_dtype, int head_dim, int num_heads, int num_kv_heads) {
+  const bool mfma = kv_dtype != PKV_F32 && (head_dim == 64 || head_dim == 128) &&
+                    PKV_DECODE_USE_MFMA;
+  return plan_tasks(num_heads, num_kv_heads, mfma);
+}
+// The plan of a one-launch cascade, which takes 8-wave workgroups only: where the wide plan
+// has fewer waves and the narrow one eight, the narrow one.
+DecodePlan plan_cascade(int kv_dtype, int head_dim, int num_heads, int num_kv_heads) {
+  const DecodePlan p = plan_decode(kv_dtype, head_dim, num_heads, num_kv_heads);
+  if (p.wpg == PKV_DECODE_WAVES_PER_WG) return p;
+  const DecodePlan n = plan_tasks(num_heads, num_kv_heads, false);
+  return n.wpg == PKV_DECODE_WAVES_PER_WG ? n : p;
+}
+
+// Workgroups of a plan that the current device holds at once (see pkv_decode_workgroups).
+int32_t plan_workgroups(const DecodePlan& p, int kv_dtype, int head_dim) {
+  int dev = 0, cus = 0, per_cu = 0, tile = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+  if (e == hipSuccess) e = by_dtype(kv_dtype, head_dim, p.gpw, QueryDecode{p.wpg, &tile, &per_cu});
+  if (e != hipSuccess) return PKV_E_HIP;
+  const int g = cus * (per_cu < 1 ? 1 : per_cu) / p.ygrid;
+  return g < 1 ? 1 : g;
 }
 
 int check_decode_shape(int kv_dtype, int head_dim, int num_heads, int num_kv_heads) {
@@ -278,7 +318,7 @@ int choose_split(int kv_dtype, int head_dim, int batch, int num_heads, int num_k
   const int st = device_cus(&cus);
   if (st) return st;
   const int groups = num_heads / num_kv_heads;
-  for (int g = 1; g <= 4; ++g)
+  for (int g = 1; g <= kWideHeads; ++g)  // past 4 heads: the wide form
     if (groups % g == 0 && (int64_t)batch * num_kv_heads * (groups / g) <= cus) {
       *gpw = g;
       break;
@@ -340,7 +380,8 @@ int decode_ex(void* out, int out_dtype, int64_t out_stride_b, int64_t out_stride
       q_stride_b % vec || q_stride_h % vec || kv_stride_slot % vec || kv_stride_head % vec ||
       out_stride_b % vec || out_stride_h % vec)
     return PKV_E_ALIGN;
-  DecodePlan p = plan_decode(num_heads, num_kv_heads);
+  DecodePlan p = one ? plan_cascade(kv_dtype, head_dim, num_heads, num_kv_heads)
+                     : plan_decode(kv_dtype, head_dim, num_heads, num_kv_heads);
   bool split = false;
   if (num_workgroups == 0) {  // the library's default split of the work
     int split_gpw = 0;
@@ -353,7 +394,7 @@ int decode_ex(void* out, int out_dtype, int64_t out_stride_b, int64_t out_stride
       p.gpw = split_gpw;
       p.nsub = num_heads / num_kv_heads / split_gpw;
     } else {
-      num_workgroups = pkv_decode_workgroups(kv_dtype, head_dim, num_heads, num_kv_heads);
+      num_workgroups = plan_workgroups(p, kv_dtype, head_dim);
       if (num_workgroups < 1) return num_workgroups < 0 ? num_workgroups : PKV_E_HIP;
     }
   }
@@ -379,6 +420,7 @@ int decode_ex(void* out, int out_dtype, int64_t out_stride_b, int64_t out_stride
   a.nkv = num_kv_heads;
   a.groups = num_heads / num_kv_heads;
   a.nsub = p.nsub;
+  a.gpw = p.gpw;
   a.bs = block_size;
   a.bs_shift = (block_size & (block_size - 1)) == 0 ? __builtin_ctz(block_size) : -1;
   int tile = 0;
@@ -459,10 +501,9 @@ int cascade_prefix_wg(int kv_dtype, int head_dim, int num_heads, int num_kv_head
                       int requested) {
   if (requested < 0 || items < 1 || check_decode_shape(kv_dtype, head_dim, num_heads, num_kv_heads))
     return 0;
-  const DecodePlan p = plan_decode(num_heads, num_kv_heads);
+  const DecodePlan p = plan_cascade(kv_dtype, head_dim, num_heads, num_kv_heads);
   if (!cascade_one_launch_shape(kv_dtype, head_dim, block_size, batch, p.wpg)) return 0;
-  if (num_workgroups == 0)
-    num_workgroups = pkv_decode_workgroups(kv_dtype, head_dim, num_heads, num_kv_heads);
+  if (num_workgroups == 0) num_workgroups = plan_workgroups(p, kv_dtype, head_dim);
   if (num_workgroups < 2) return 0;
   int64_t wg = requested;
   if (wg == 0) {
@@ -491,14 +532,8 @@ int32_t pkv_decode_workgroups(int kv_dtype, int32_t head_dim, int32_t num_heads,
                               int32_t num_kv_heads) {
   const int bad = check_decode_shape(kv_dtype, head_dim, num_heads, num_kv_heads);
   if (bad) return bad;
-  const DecodePlan p = plan_decode(num_heads, num_kv_heads);
-  int dev = 0, cus = 0, per_cu = 0, tile = 0;
-  hipError_t e = hipGetDevice(&dev);
-  if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-  if (e == hipSuccess) e = by_dtype(kv_dtype, head_dim, p.gpw, QueryDecode{p.wpg, &tile, &per_cu});
-  if (e != hipSuccess) return PKV_E_HIP;
-  const int g = cus * (per_cu < 1 ? 1 : per_cu) / p.ygrid;
-  return g < 1 ? 1 : g;
+  return plan_workgroups(plan_decode(kv_dtype, head_dim, num_heads, num_kv_heads), kv_dtype,
+                         head_dim);
 }
 
 int32_t pkv_decode_default_workgroups(int kv_dtype, int32_t head_dim, int32_t num_heads,

@@ -21,6 +21,7 @@ struct DecodeArgs {
   int32_t max_blocks;
   const int32_t* ctx;
   int32_t batch, nh, nkv, groups, nsub, bs, bs_shift;  // bs_shift < 0: block_size not pow2
+  int32_t gpw;          // query heads per wave (groups / nsub)
   int32_t unit_tokens;  // TILE of the instantiated kernel
   int32_t num_wg;       // unit ranges (workgroups along x) sharing the unit stream
   // One-launch cascade (kernels instantiated with WT): the stream is cut into `slots`
@@ -542,9 +543,24 @@ paged_decode_stream_kernel(const DecodeArgs a) {
 //     to the whole row), since token 4g + r's score sits in lane (h, g) of that row.
 // When block_size is a multiple of 16 a tile lies inside one block: its block id is
 // read with v_readlane into a scalar and every lane's address is a fixed offset from it.
+//
+// GPW = kWideHeads (groups of 5 to 16 query heads): the score tile has 16 columns, so one
+// wave takes up to 16 query heads (a.gpw of them) for the same K reads and MFMAs, and
+// P.V moves to the matrix cores too (its accumulator O^T, 4 VGPRs per 16 dims, does not
+// grow with the heads either). Split over waves of at most 4 heads, a group's K and V
+// went through L2 once per wave, and a group of 5 or 7 took one head per wave: 48 sequences
+// of 256-4,096 tokens, 8 KV heads, hd 128, groups of 5 / 6 / 8: 288 / 121 / 123 us per call,
+// now 75.8 / 77.1 / 78.2 (5.4 TB/s): bound by HBM as the narrow form is. Small batches take
+// it in the split pass (20 sequences of 1-600 tokens, groups of 8: 19.9 -> 15.0 us).
 // ---------------------------------------------------------------------------------
 
-
+constexpr int kWideHeads = 16;  // query heads a wave of the wide instantiations may hold
+// Whether the stream pass runs P.V on the matrix cores, and the LDS each of its waves then
+// stages V rows in (8 KB per step of K and V: 4 KB of V).
+template <int HD, int GPW, bool SPLIT = false> constexpr bool pv_mfma() {
+  return GPW > 4 || (HD == 64 && !SPLIT && PKV_DECODE_PV_MFMA);
+}
+constexpr int kVSlotBytes = 4096;
 
 template <int DT> struct Mfma16x16x32;
 template <> struct Mfma16x16x32<PKV_BF16> {
@@ -563,6 +579,53 @@ template <> struct Mfma16x16x32<PKV_F16> {
                                                   __builtin_bit_cast(v8, b), c, 0, 0, 0);
   }
 };
+
+// Four probabilities per lane against four V rows: v_mfma_f32_16x16x16, the contraction
+// of one 16-token tile. P enters as TERMS 16-bit terms, each the rounded rest of the ones
+// before it: bf16 takes three (24 bits, what fp32 P has), fp16 two (22 bits; the caller
+// scales P by 2^7, so weights down to 2^-32 of the largest keep a part).
+template <int DT> struct Mfma16x16x16;
+template <> struct Mfma16x16x16<PKV_BF16> {
+  static constexpr int TERMS = 3;
+  typedef __bf16 v2 __attribute__((ext_vector_type(2)));
+  __device__ static uint32_t pack(float x, float y) {
+    return __builtin_bit_cast(uint32_t, v2{(__bf16)x, (__bf16)y});
+  }
+  __device__ static float low(uint32_t w) { return __uint_as_float(w << 16); }
+  __device__ static float high(uint32_t w) { return __uint_as_float(w & 0xFFFF0000u); }
+  __device__ static f32x4 mma(s16x4 a, s16x4 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0);
+  }
+};
+template <> struct Mfma16x16x16<PKV_F16> {
+  static constexpr int TERMS = 2;
+  typedef _Float16 v2 __attribute__((ext_vector_type(2)));
+  typedef _Float16 v4 __attribute__((ext_vector_type(4)));
+  __device__ static uint32_t pack(float x, float y) {
+    return __builtin_bit_cast(uint32_t, v2{(_Float16)x, (_Float16)y});
+  }
+  __device__ static float low(uint32_t w) { return (float)__builtin_bit_cast(v2, w)[0]; }
+  __device__ static float high(uint32_t w) { return (float)__builtin_bit_cast(v2, w)[1]; }
+  __device__ static f32x4 mma(s16x4 a, s16x4 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(v4, a),
+                                                 __builtin_bit_cast(v4, b), c, 0, 0, 0);
+  }
+};
+// Probabilities p[0 .. 3] as the terms' operand fragments.
+template <int DT>
+__device__ __forceinline__ void pack_terms(const float* p, s16x4 (&t)[Mfma16x16x16<DT>::TERMS]) {
+  using M = Mfma16x16x16<DT>;
+  float r[4] = {p[0], p[1], p[2], p[3]};
+#pragma unroll
+  for (int n = 0; n < M::TERMS; ++n) {
+    uint2 w = make_uint2(M::pack(r[0], r[1]), M::pack(r[2], r[3]));
+    // the empty asm keeps the packed pair one value (no second conversion for the rest)
+    __asm__("" : "+v"(w.x), "+v"(w.y));
+    t[n] = __builtin_bit_cast(s16x4, w);
+    r[0] -= M::low(w.x), r[1] -= M::high(w.x);
+    r[2] -= M::low(w.y), r[3] -= M::high(w.y);
+  }
+}
 
 __device__ __forceinline__ u32x4 load_kv16v(const void* p) {
 #if PKV_DECODE_STREAM_LOADS
@@ -647,10 +710,66 @@ __device__ __forceinline__ void split_merge(const DecodeArgs& a, int b, int h0,
   }
 }
 
+// The same for the wide form, whose states are O^T (head col's dims 16 d + 4 grp .. + 3 in
+// lane (col, grp)): kSplitWaves heads at a time through the V slots (free once every wave has
+// passed its last tile), head g0 + w merged by wave w. ng is the workgroup's.
+template <int DT, int HD>
+__device__ __forceinline__ void split_merge_wide(const DecodeArgs& a, int b, int h0, int ng,
+                                                 const f32x4 (&ov)[HD / 16], float o_scale,
+                                                 float l_own, float m_own, u32x4* vslots) {
+  constexpr int W = kSplitWaves, DPL = HD / kWave;
+  static_assert(W * HD * 4 <= kVSlotBytes, "a round of heads fits the V slots");
+  using S = typename Elt<DT>::S;
+  __shared__ float part_ml[W][kWideHeads][2];
+  float* const part = reinterpret_cast<float*>(vslots);  // [wave][head of the round][HD]
+  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+  const int col = lane & 15, grp = lane >> 4;
+  if (grp == 0 && col < ng) {
+    part_ml[wave][col][0] = m_own;
+    part_ml[wave][col][1] = l_own;
+  }
+  for (int g0 = 0; g0 < ng; g0 += W) {
+    __syncthreads();
+    if (col >= g0 && col < min(ng, g0 + W)) {
+#pragma unroll
+      for (int d = 0; d < HD / 16; ++d)
+        *reinterpret_cast<f32x4*>(part + (wave * W + col - g0) * HD + 16 * d + 4 * grp) = ov[d] * o_scale;
+    }
+    __syncthreads();
+    const int g = g0 + wave;
+    if (g >= ng) continue;
+    float mmax = -INFINITY;
+#pragma unroll
+    for (int s = 0; s < W; ++s) mmax = fmaxf(mmax, part_ml[s][g][0]);
+    const float mref = mmax == -INFINITY ? 0.f : mmax;  // nothing live: weights 0
+    float l = 0.f, o[DPL];
+#pragma unroll
+    for (int k = 0; k < DPL; ++k) o[k] = 0.f;
+#pragma unroll
+    for (int s = 0; s < W; ++s) {
+      const float wgt = __builtin_amdgcn_exp2f(part_ml[s][g][0] - mref);  // empty share: 0
+      l = __builtin_fmaf(wgt, part_ml[s][g][1], l);
+#pragma unroll
+      for (int k = 0; k < DPL; ++k)
+        o[k] = __builtin_fmaf(wgt, part[(s * W + wave) * HD + DPL * lane + k], o[k]);
+    }
+    const float inv = l > 0.f ? 1.f / l : 0.f;  // empty context: 0
+    const int64_t e = b * a.out_sb + (int64_t)(h0 + g) * a.out_sh + DPL * lane;
+#pragma unroll
+    for (int k = 0; k < DPL; ++k) {
+      const float v = o[k] * inv;
+      if (a.out_f32) reinterpret_cast<float*>(a.out)[e + k] = v;
+      else reinterpret_cast<S*>(a.out)[e + k] = Elt<DT>::from_f32(v);
+    }
+  }
+}
+
 // The MFMA stream pass of workgroup (bx, by): bx indexes the unit ranges (or, SPLIT, the
-// sequence), by the task group.
+// sequence), by the task group. vslots: kVSlotBytes of LDS per wave where P.V runs on the
+// matrix cores (pv_mfma), else unused.
 template <int DT, int GPW, bool FAST, int HD, bool SPLIT, bool STAGED = false, bool WT = false>
-__device__ __forceinline__ void decode_mfma_body(const DecodeArgs& a, const int bx, const int by) {
+__device__ __forceinline__ void decode_mfma_body(const DecodeArgs& a, const int bx, const int by,
+                                                 u32x4* const vslots) {
   static_assert(!WT || STAGED, "the one-launch cascade's split takes the staged pass");
   // hd 128: a step is one 16-token tile, four 32-dim MFMA k-blocks, V rows over all 16
   // lane columns (8 dims each). hd 64: a step is two 16-token sub-tiles (the same 8 KB
@@ -659,9 +778,13 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeArgs& a, const int 
   static_assert(HD == 64 || HD == 128, "MFMA decode: hd 64 or 128");
   constexpr int TILE = 16, KB = HD / 32, VC = HD / 8, NS = 128 / HD, STEP = NS * TILE;
   constexpr bool kDeep = PKV_DECODE_PREFETCH >= 2;
-  static_assert(GPW >= 1 && GPW <= 4, "at most 4 query heads per wave");
+  constexpr bool WIDE = GPW > 4;
+  static_assert(GPW >= 1 && (GPW <= 4 || GPW == kWideHeads),
+                "at most 4 query heads per wave, or the wide form");
+  const int ng = WIDE ? a.gpw : GPW;  // query heads of this wave
   using S = typename Elt<DT>::S;
   using MMA = Mfma16x16x32<DT>;
+  using MMA4 = Mfma16x16x16<DT>;
   // hd 64: P.V on the matrix cores (PKV_DECODE_PV_MFMA; 5.6% faster than the VALU form,
   // a row broadcast and 8 FMAs per query head and V row, at config 2's batch and
   // contexts; at hd 128, a timing copy without any P.V ran only 1% faster, so it keeps
@@ -673,9 +796,10 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeArgs& a, const int 
   // grp) holds dims 16 d + 4 grp + r.
   // (The stream-K pass only: the split pass's few short steps per wave are latency-bound,
   // and the LDS round trip cost config 1 0.2 us.)
-  constexpr bool PVM = HD == 64 && !SPLIT && PKV_DECODE_PV_MFMA;
-  __shared__ __align__(16) u32x4 v_lds[PVM ? PKV_DECODE_WAVES_PER_WG * 256 : 1];
-  char* const vslot = reinterpret_cast<char*>(&v_lds[PVM ? (threadIdx.x / kWave) * 256 : 0]);
+  // hd 128, wide: the same with one 16-token tile per step (4 KiB of V) and 16x16x16
+  // MFMAs, P in fp32-like terms (pack_terms), as the VALU form it replaces had fp32 P.
+  constexpr bool PVM = pv_mfma<HD, GPW, SPLIT>();
+  char* const vslot = reinterpret_cast<char*>(vslots) + (PVM ? (threadIdx.x / kWave) * kVSlotBytes : 0);
 
   const int lane = threadIdx.x & (kWave - 1);
   // Stream-K: wave = task (KV head and head sub-group), workgroup x = unit range.
@@ -684,7 +808,7 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeArgs& a, const int 
                          : (int)(by * (blockDim.x / kWave) + (threadIdx.x / kWave));
   const int kvh = task / a.nsub;
   if (!SPLIT && !STAGED && kvh >= a.nkv) return;
-  const int h0 = kvh * a.groups + (task - kvh * a.nsub) * GPW;
+  const int h0 = kvh * a.groups + (task - kvh * a.nsub) * ng;
   // Unit range of this workgroup, XCD-blocked when the grid is a multiple of 8:
   // workgroups are dealt to the 8 XCDs round-robin, so workgroup bx (XCD bx % 8) takes
   // range (bx % 8) G / 8 + bx / 8, and each XCD streams one contiguous eighth of the
@@ -776,7 +900,7 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeArgs& a, const int 
       const S* qp = reinterpret_cast<const S*>(a.q) + b * a.q_sb + (int64_t)(h0 + col) * a.q_sh + 8 * grp;
 #pragma unroll
       for (int m = 0; m < KB; ++m)
-        qb[m] = col < GPW ? *reinterpret_cast<const u32x4*>(qp + 32 * m) : u32x4{0, 0, 0, 0};
+        qb[m] = col < ng ? *reinterpret_cast<const u32x4*>(qp + 32 * m) : u32x4{0, 0, 0, 0};
     }
 
     int cb = 0, tbl = 0;
@@ -950,16 +1074,17 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeArgs& a, const int 
       else return load_pair(tb, kr, vr);
     };
 
-    float m_run = -INFINITY;  // exponent reference of head column col (same in all 4 rows)
-    float l_run = 0.f;        // this row's share of the running sum
-    float acc[GPW][8];
-#pragma unroll
-    for (int g = 0; g < GPW; ++g)
-#pragma unroll
-      for (int d = 0; d < 8; ++d) acc[g][d] = 0.f;
-    f32x4 ov[PVM ? 4 : 1];  // PVM: O^T, dims 16 d .. 16 d + 15
-#pragma unroll
-    for (int d = 0; d < (PVM ? 4 : 1); ++d) ov[d] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float m_run;  // exponent reference of head column col (same in all 4 rows)
+    float l_run;  // this row's share of the running sum
+    constexpr int NACC = PVM ? 1 : GPW, NOV = PVM ? HD / 16 : 1;
+    float acc[NACC][8];  // VALU P.V
+    f32x4 ov[NOV];       // PVM: O^T, dims 16 d .. 16 d + 15
+    // PVM at hd 128: whether the tiles keep infinities and NaNs of V out of P's lower terms.
+    // A term can be 0 where P is not, and 0 x inf would turn an infinite output into NaN: a
+    // piece that ends with a NaN runs a second time with them kept out (V is finite in
+    // practice, so the first run is free of the checks).
+    constexpr bool kTerms = PVM && NS == 1;
+    bool v_careful = false;
 
     // The exponent reference of head column col is raised only when a tile's maximum
     // exceeds it by more than 2^8 (or it is still -inf): a stale reference changes
@@ -976,7 +1101,7 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeArgs& a, const int 
         l_run *= alpha;
         if constexpr (PVM) {  // O^T column col is head col: its own factor
 #pragma unroll
-          for (int d = 0; d < 4; ++d) ov[d] *= alpha;
+          for (int d = 0; d < NOV; ++d) ov[d] *= alpha;
         } else {
 #pragma unroll
           for (int g = 0; g < GPW; ++g) {
@@ -990,6 +1115,25 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeArgs& a, const int 
     };
     auto tile = [&](const u32x4* kr, const u32x4* vr, unsigned ok) {
       if constexpr (NS == 1) {
+        // PVM: V row 4 grp + r goes to the wave's slot, chunk col at (col ^ swz(row)), swz(t)
+        // = (t3, t0, t1, t2) as in the prefill's tiles, and comes back as V^T fragments:
+        // lane (dim 16 d + col, grp) gets tokens 4 grp .. + 3 (see the hd-64 form below).
+        s16x4 vt4[PVM ? NOV : 1];
+        if constexpr (PVM) {
+          auto swz = [](int t) { return ((t & 7) << 1) | ((t >> 3) & 1); };
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int tk = 4 * grp + r;
+            *reinterpret_cast<u32x4*>(vslot + tk * 256 + ((col ^ swz(tk)) << 4)) = vr[r];
+          }
+          const int c4 = col & 3, tr = 4 * grp + (col >> 2);
+#pragma unroll
+          for (int d = 0; d < NOV; ++d) {
+            const int off = tr * 256 + (((2 * d + (c4 >> 1)) ^ swz(tr)) << 4) + ((c4 & 1) << 3);
+            vt4[d] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(vslot + off));
+          }
+          __builtin_amdgcn_sched_barrier(0);  // the reads stay ahead of the scores
+        }
         f32x4 s = {0.f, 0.f, 0.f, 0.f};
   #pragma unroll
         for (int m = 0; m < KB; ++m) s = MMA::mma(kr[m], qb[m], s);
@@ -1004,6 +1148,28 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeArgs& a, const int 
   #pragma unroll
         for (int r = 0; r < 4; ++r) p[r] = __builtin_amdgcn_exp2f(p[r] - mref);
         l_run += (p[0] + p[1]) + (p[2] + p[3]);
+        if constexpr (PVM) {
+          if constexpr (DT == PKV_F16) {  // scaled as in the hd-64 form below
+#pragma unroll
+            for (int r = 0; r < 4; ++r) p[r] *= 128.f;
+          }
+          s16x4 pt[MMA4::TERMS];
+          pack_terms<DT>(p, pt);
+#pragma unroll
+          for (int d = 0; d < NOV; ++d) ov[d] = MMA4::mma(vt4[d], pt[0], ov[d]);
+          if (v_careful) {  // wave-uniform
+            constexpr short kExp = DT == PKV_BF16 ? 0x7F80 : 0x7C00;
+#pragma unroll
+            for (int d = 0; d < NOV; ++d)
+#pragma unroll
+              for (int e = 0; e < 4; ++e)
+                if ((vt4[d][e] & kExp) == kExp) vt4[d][e] = 0;
+          }
+#pragma unroll
+          for (int n = 1; n < MMA4::TERMS; ++n)
+#pragma unroll
+            for (int d = 0; d < NOV; ++d) ov[d] = MMA4::mma(vt4[d], pt[n], ov[d]);
+        } else {
         float vf[4][8];
   #pragma unroll
         for (int r = 0; r < 4; ++r) unpack16v<DT>(vr[r], vf[r]);
@@ -1015,6 +1181,7 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeArgs& a, const int 
   #pragma unroll
             for (int d = 0; d < 8; ++d) acc[g][d] = __builtin_fmaf(pr, vf[r][d], acc[g][d]);
           }
+        }
         }
       } else {
         // PVM: the step's V goes through the wave's LDS slot first, so the transpose
@@ -1104,6 +1271,15 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeArgs& a, const int 
       }
     };
 
+    for (int run = 0; run < (kTerms ? 2 : 1); ++run) {
+    m_run = -INFINITY;
+    l_run = 0.f;
+#pragma unroll
+    for (int g = 0; g < NACC; ++g)
+#pragma unroll
+      for (int d = 0; d < 8; ++d) acc[g][d] = 0.f;
+#pragma unroll
+    for (int d = 0; d < NOV; ++d) ov[d] = f32x4{0.f, 0.f, 0.f, 0.f};
     if (t0 < t1) {
       load_table(block_of(t0));
       if constexpr (kDeep) {
@@ -1135,34 +1311,58 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeArgs& a, const int 
         }
       }
     }
+    if constexpr (kTerms) {
+      bool nan = false;
+#pragma unroll
+      for (int d = 0; d < NOV; ++d)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) nan = nan || ov[d][r] != ov[d][r];
+      v_careful = __builtin_amdgcn_ballot_w64(nan && col < ng) != 0;
+      if (!v_careful) break;
+    }
+    }
 
     // Totals: l over the four rows of each column, acc over the four rows (and, at hd 64,
     // over the two sub-tiles' lane columns c and c + 8, which hold the same dims).
     const float l_tot = rows_sum(l_run);
     if constexpr (PVM) {
-      // O^T (already summed over every token) to acc's layout below -- lanes grp 0, col
-      // < 8: head g's dims 8 col .. 8 col + 7 -- through the wave's slot, after the last
-      // step's reads of it (LDS keeps one wave's accesses in order).
-      float* xs = reinterpret_cast<float*>(vslot);  // [GPW][64]
+      // O^T is summed over every token already: lane (head col, grp) holds dims 16 d + 4
+      // grp .. + 3 of head h0 + col, and stores them as they are.
       constexpr float kOScale = DT == PKV_F16 ? 1.f / 128.f : 1.f;  // P's fp16 scale undone
-      if (col < GPW) {
-#pragma unroll
-        for (int d = 0; d < 4; ++d)
-          *reinterpret_cast<f32x4*>(xs + col * 64 + 16 * d + 4 * grp) = ov[d] * kOScale;
+      if constexpr (SPLIT) {
+        split_merge_wide<DT, HD>(a, b, h0, ng, ov, kOScale, l_tot, m_run, vslots);
+        return;
       }
+      if (col < ng) {
+        if (whole) {
+          const WholeDst dst = whole_dst(a, pre_b);
+          const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
+          const int64_t e = b * dst.sb + (int64_t)(h0 + col) * dst.sh + 4 * grp;
 #pragma unroll
-      for (int g = 0; g < GPW; ++g)
+          for (int d = 0; d < NOV; ++d) {
+            const f32x4 o4 = ov[d] * kOScale * inv;
+            const float o[4] = {o4[0], o4[1], o4[2], o4[3]};
+            if (dst.f32) store_vec<PKV_F32, 4>((float*)dst.p + e + 16 * d, o);
+            else store_vec<DT, 4>((S*)dst.p + e + 16 * d, o);
+          }
+          if (dst.lse && grp == 0) dst.lse[(int64_t)b * a.nh + h0 + col] = lse_of(m_run, l_tot);
+        } else {
+          const int64_t rec = ((int64_t)w * 2 + slot) * a.nh + h0 + col;
 #pragma unroll
-        for (int d = 0; d < 8; ++d) acc[g][d] = (grp == 0 && col < 8) ? xs[g * 64 + 8 * col + d] : 0.f;
+          for (int d = 0; d < NOV; ++d)
+            *reinterpret_cast<f32x4*>(a.ws_acc + rec * HD + 16 * d + 4 * grp) = ov[d] * kOScale;
+          if (grp == 0) *reinterpret_cast<float2*>(a.ws_ml + 2 * rec) = make_float2(m_run, l_tot);
+        }
+      }
+      continue;
     } else {
 #pragma unroll
-      for (int g = 0; g < GPW; ++g)
+    for (int g = 0; g < GPW; ++g)
 #pragma unroll
-        for (int d = 0; d < 8; ++d) {
-          acc[g][d] = rows_sum(acc[g][d]);
-          if constexpr (NS == 2) acc[g][d] += dpp<kRowRor8>(acc[g][d]);  // lanes c, c ^ 8
-        }
-    }
+      for (int d = 0; d < 8; ++d) {
+        acc[g][d] = rows_sum(acc[g][d]);
+        if constexpr (NS == 2) acc[g][d] += dpp<kRowRor8>(acc[g][d]);  // lanes c, c ^ 8
+      }
     float lh[GPW], mh[GPW];
 #pragma unroll
     for (int g = 0; g < GPW; ++g) {
@@ -1198,13 +1398,17 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeArgs& a, const int 
         }
       }
     }
+    }
   }
 }
 
+// Dynamic LDS: kVSlotBytes per wave where P.V runs on the matrix cores (pv_mfma).
 template <int DT, int GPW, bool FAST, int HD, bool SPLIT, bool STAGED = false>
 __global__ void __launch_bounds__(512)
 paged_decode_mfma_kernel(const DecodeArgs a) {
-  decode_mfma_body<DT, GPW, FAST, HD, SPLIT, STAGED>(a, (int)blockIdx.x, (int)blockIdx.y);
+  extern __shared__ __align__(16) u32x4 decode_vslots[];
+  decode_mfma_body<DT, GPW, FAST, HD, SPLIT, STAGED>(a, (int)blockIdx.x, (int)blockIdx.y,
+                                                     decode_vslots);
 }
 
 // ---------------------------------------------------------------------------------

@@ -1094,8 +1094,8 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs& a, const Prefill
 // items on one workgroup puts a barrier between them (the merge reuses the rings).
 // V16: V from the fp16 copy (bf16 caches; the launch guarantees every chunk's region).
 template <int DT, int HD, bool POW2, bool V16 = false>
-__device__ __forceinline__ void prefill_item(const PrefillArgs& a, const int item) {
-  __shared__ __align__(16) PrefillLds<HD> lds;
+__device__ __forceinline__ void prefill_item(const PrefillArgs& a, const int item,
+                                             PrefillLds<HD>& lds) {
   const int lane = threadIdx.x & (kWave - 1);
   // Work items (chunk, row block, KV head), heaviest first: chunks by context length
   // (longest first), then row blocks from the last (it sees the most keys), KV heads
@@ -1134,7 +1134,8 @@ __device__ __forceinline__ void prefill_item(const PrefillArgs& a, const int ite
 template <int DT, int HD, bool POW2, bool V16>
 __global__ void __launch_bounds__(512)
 paged_prefill_kernel(const PrefillArgs a) {
-  prefill_item<DT, HD, POW2, V16>(a, (int)blockIdx.x);
+  __shared__ __align__(16) PrefillLds<HD> lds;
+  prefill_item<DT, HD, POW2, V16>(a, (int)blockIdx.x, lds);
 }
 
 // The fp16 copy of the chunks' V for the bf16 matrix-core prefill (PrefillArgs::v16):
