@@ -171,6 +171,26 @@ int pkv_paged_decode_noalloc(void* out, int out_dtype, int64_t out_stride_b,
                              int32_t num_kv_heads, int32_t head_dim, int32_t block_size,
                              float scale, int32_t num_workgroups, void* stream);
 
+/*
+ * pkv_paged_decode on rows of larger q and out tensors: sequence b's query is row rows[b]
+ * (device int64 [batch]; NULL: b) of q, and its result goes to the same row of out; both hold
+ * num_rows rows. Negative values count from the end; a sequence whose row lies outside
+ * [0, num_rows) is skipped, rows that no sequence names are left as they are, and of
+ * sequences that name one row one's result stays. Replaces the gather and scatter around the
+ * decode rows of a mixed step (reference engine/model/layers.py:227-245). out may be q itself
+ * (same strides).
+ */
+int pkv_paged_decode_rows(void* out, int out_dtype, int64_t out_stride_b, int64_t out_stride_h,
+                          const void* q, int64_t q_stride_b, int64_t q_stride_h,
+                          const void* k_cache, const void* v_cache, int kv_dtype,
+                          int64_t kv_stride_slot, int64_t kv_stride_head, int64_t num_slots,
+                          const int32_t* block_tables, int64_t table_stride, int32_t max_blocks,
+                          const int32_t* context_lens, int32_t batch, int32_t num_heads,
+                          int32_t num_kv_heads, int32_t head_dim, int32_t block_size,
+                          float scale, int32_t num_workgroups, void* workspace,
+                          int64_t workspace_bytes, const int64_t* rows, int64_t num_rows,
+                          void* stream);
+
 /* Bytes of scratch pkv_paged_decode_ex needs with prefix parts (cascade): the split-K
  * scratch plus fp32 room for the sequences the stream pass finishes, [batch, num_heads,
  * head_dim + 1]. Needed at any num_workgroups, 1 included. */
@@ -333,6 +353,25 @@ int pkv_paged_prefill_ws(void* out, int out_dtype, int64_t out_stride_tok, int64
                          int32_t n_chunks, int32_t max_query_len, int32_t num_heads,
                          int32_t num_kv_heads, int32_t head_dim, int32_t block_size, float scale,
                          void* workspace, int64_t workspace_bytes, void* stream);
+
+/*
+ * pkv_paged_prefill_ws on rows of larger q and out tensors: query token t of the step (the
+ * positions cu_seqlens_q counts) is row rows[t] (device int64 [rows_len]; NULL: t) of q, and
+ * its result goes to the same row of out; both hold num_rows rows (below 2^31). Rows as in
+ * pkv_paged_decode_rows; tokens at rows_len or beyond are skipped. Replaces the gather and
+ * scatter around the chunk rows of a mixed step (reference engine/model/layers.py:246-253).
+ */
+int pkv_paged_prefill_rows(void* out, int out_dtype, int64_t out_stride_tok, int64_t out_stride_h,
+                           const void* q, int64_t q_stride_tok, int64_t q_stride_h,
+                           const void* k_cache, const void* v_cache, int kv_dtype,
+                           int64_t kv_stride_slot, int64_t kv_stride_head, int64_t num_slots,
+                           const int32_t* block_tables, int64_t table_stride, int32_t max_blocks,
+                           const int32_t* context_lens, const int32_t* cu_seqlens_q,
+                           int32_t n_chunks, int32_t max_query_len, int32_t num_heads,
+                           int32_t num_kv_heads, int32_t head_dim, int32_t block_size,
+                           float scale, void* workspace, int64_t workspace_bytes,
+                           const int64_t* rows, int64_t rows_len, int64_t num_rows,
+                           void* stream);
 
 /*
  * Fused element-wise kernels (csrc/fused.hip). Replace the reference's Triton kernels of

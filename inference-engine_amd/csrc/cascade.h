@@ -34,7 +34,7 @@ struct CascadeLaunch {
   int wslots, tail_slots;
 };
 
-// decode.hip: pkv_paged_decode_ex; with `one`, the stream pass runs in one launch with
+// decode.hip: pkv_paged_decode_ex (rows, num_rows: pkv_paged_decode_rows); with `one`, the stream pass runs in one launch with
 // the prefix pass `one` describes (PKV_E_SHAPE where cascade_prefix_wg gives 0). With
 // check_only, every argument check runs and nothing is launched.
 int decode_ex(void* out, int out_dtype, int64_t out_stride_b, int64_t out_stride_h,
@@ -47,7 +47,7 @@ int decode_ex(void* out, int out_dtype, int64_t out_stride_b, int64_t out_stride
               const int32_t* first_block, float* lse, const float* prefix_out,
               const float* prefix_lse, const int32_t* prefix_row, int32_t prefix_parts,
               int64_t prefix_stride, void* stream, const CascadeLaunch* one,
-              bool check_only);
+              bool check_only, const int64_t* rows = nullptr, int64_t num_rows = 0);
 
 // decode.hip: the prefix workgroups of a one-launch cascade for these shapes with `items`
 // prefix items (requested > 0: that many; 0: the library's choice), or 0 when the call

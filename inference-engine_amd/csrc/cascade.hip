@@ -44,7 +44,7 @@ cascade_decode_kernel(const DecodeArgs d, const PrefillArgs p, const int prefix_
   if (bx < prefix_wg) {
     const int workers = prefix_wg * (int)gridDim.y;
     for (int it = (int)blockIdx.y * prefix_wg + bx; it < items; it += workers) {
-      prefill_item<DT, HD, true>(p, it, lds);
+      prefill_item<DT, HD, true, false, false>(p, it, lds);
       __syncthreads();  // the item's merge used the rings the next item's loads fill
     }
     if (d.num_wg == d.full_wg) return;  // no stream share for prefix workgroups
@@ -67,18 +67,18 @@ hipError_t launch_hd(const DecodeArgs& d, PrefillArgs p, int64_t rows, int gpw, 
     return hipErrorInvalidValue;
   const dim3 grid((unsigned)gx, (unsigned)ygrid), block(512);
   const int n = (int)items;
-  switch (gpw) {
+  switch (pv_mfma<HD, 1>() ? kWideHeads : gpw) {
     case 1:
-      hipLaunchKernelGGL((cascade_decode_kernel<DT, 1, HD>), grid, block, 0, st, d, p, prefix_wg, n);
+      hipLaunchKernelGGL((cascade_decode_kernel<DT, stream_gpw<HD, 1>(), HD>), grid, block, 0, st, d, p, prefix_wg, n);
       break;
     case 2:
-      hipLaunchKernelGGL((cascade_decode_kernel<DT, 2, HD>), grid, block, 0, st, d, p, prefix_wg, n);
+      hipLaunchKernelGGL((cascade_decode_kernel<DT, stream_gpw<HD, 2>(), HD>), grid, block, 0, st, d, p, prefix_wg, n);
       break;
     case 3:
-      hipLaunchKernelGGL((cascade_decode_kernel<DT, 3, HD>), grid, block, 0, st, d, p, prefix_wg, n);
+      hipLaunchKernelGGL((cascade_decode_kernel<DT, stream_gpw<HD, 3>(), HD>), grid, block, 0, st, d, p, prefix_wg, n);
       break;
     case 4:
-      hipLaunchKernelGGL((cascade_decode_kernel<DT, 4, HD>), grid, block, 0, st, d, p, prefix_wg, n);
+      hipLaunchKernelGGL((cascade_decode_kernel<DT, stream_gpw<HD, 4>(), HD>), grid, block, 0, st, d, p, prefix_wg, n);
       break;
     default:
       hipLaunchKernelGGL((cascade_decode_kernel<DT, kWideHeads, HD>), grid, block, 0, st, d, p,

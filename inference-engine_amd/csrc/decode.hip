@@ -85,7 +85,8 @@ template <class F> hipError_t by_dtype(int dt, int hd, int gpw, const F& f) {
 
 template <int DT, int HD, int GPW> const void* decode_kernel() {
   if constexpr (use_mfma<DT, HD>())
-    return reinterpret_cast<const void*>(&paged_decode_mfma_kernel<DT, GPW, true, HD, false>);
+    return reinterpret_cast<const void*>(
+        &paged_decode_mfma_kernel<DT, stream_gpw<HD, GPW>(), true, HD, false>);
   else
     return reinterpret_cast<const void*>(&paged_decode_stream_kernel<DT, HD, GPW>);
 }
@@ -106,30 +107,46 @@ template <int DT, int HD, int GPW> constexpr unsigned stream_lds(int wpg) {
 //   1,024 pairs (64 of 200-3,000, 16 heads)         71.3 / 71.4 / 72.1 / 74.6 / 77.9
 //   1,024 pairs (32 of 128-32,768, log)            106.9 / 105.7 / 105.0 / 106.5 / 110.1
 //   1,536 pairs (64 of 1,024-4,096, 24 heads)      109.8 / 110.0 / 111.6 / 115.0 / 119.8
-int combine_waves(int pairs) {
+// At 1,024 pairs four waves pay where sequences have many pieces (8 or more ranges each).
+int combine_waves(const DecodeArgs& a) {
+  const int pairs = a.batch * a.nh;
   if (pairs <= 64) return 16;
   if (pairs <= 256) return 8;
   if (pairs <= 512) return 4;
-  return pairs <= PKV_DECODE_COMBINE_SPLIT_PAIRS ? 2 : 1;
+  if (pairs > PKV_DECODE_COMBINE_SPLIT_PAIRS) return 1;
+  return a.num_wg >= 8 * a.batch ? 4 : 2;
 }
-template <int DT, int HD, int SP, bool WT>
+template <int DT, int HD, int SP, bool WT, bool ROWS>
 void launch_combine_sp(const DecodeArgs& a, hipStream_t st) {
   constexpr int WG = SP > 4 ? SP : 4;  // waves per workgroup
   const int pairs = a.batch * a.nh;
-  hipLaunchKernelGGL((paged_decode_combine_kernel<DT, HD, SP, WT>),
+  hipLaunchKernelGGL((paged_decode_combine_kernel<DT, HD, SP, WT, ROWS>),
                      dim3((unsigned)((pairs + WG / SP - 1) / (WG / SP))), dim3(kWave * WG), 0, st, a);
 }
-template <int DT, int HD, bool WT> void launch_combine(const DecodeArgs& a, hipStream_t st) {
-  switch (combine_waves(a.batch * a.nh)) {
-    case 16: return launch_combine_sp<DT, HD, 16, WT>(a, st);
-    case 8: return launch_combine_sp<DT, HD, 8, WT>(a, st);
-    case 4: return launch_combine_sp<DT, HD, 4, WT>(a, st);
-    case 2: return launch_combine_sp<DT, HD, 2, WT>(a, st);
-    default: return launch_combine_sp<DT, HD, 1, WT>(a, st);
+template <int DT, int HD, bool WT, bool ROWS>
+void launch_combine(const DecodeArgs& a, hipStream_t st) {
+  switch (combine_waves(a)) {
+    case 16: return launch_combine_sp<DT, HD, 16, WT, ROWS>(a, st);
+    case 8: return launch_combine_sp<DT, HD, 8, WT, ROWS>(a, st);
+    case 4: return launch_combine_sp<DT, HD, 4, WT, ROWS>(a, st);
+    case 2: return launch_combine_sp<DT, HD, 2, WT, ROWS>(a, st);
+    default: return launch_combine_sp<DT, HD, 1, WT, ROWS>(a, st);
   }
 }
 
 struct LaunchDecode {
+  template <int DT, int HD, int GPW, bool ROWS>
+  void launch_stream(dim3 grid, dim3 block, unsigned lds, bool staged) const {
+    constexpr int G = stream_gpw<HD, GPW>();
+    if (a->bs % 16 == 0 && staged)
+      hipLaunchKernelGGL((paged_decode_mfma_kernel<DT, G, true, HD, false, true, ROWS>), grid, block, lds, st, *a);
+    else if (a->bs % 16 == 0)
+      hipLaunchKernelGGL((paged_decode_mfma_kernel<DT, G, true, HD, false, false, ROWS>), grid, block, lds, st, *a);
+    else if (staged)
+      hipLaunchKernelGGL((paged_decode_mfma_kernel<DT, G, false, HD, false, true, ROWS>), grid, block, lds, st, *a);
+    else
+      hipLaunchKernelGGL((paged_decode_mfma_kernel<DT, G, false, HD, false, false, ROWS>), grid, block, lds, st, *a);
+  }
   const DecodeArgs* a;
   int wpg, ygrid;
   hipStream_t st;
@@ -143,14 +160,11 @@ struct LaunchDecode {
         const hipError_t e = launch_cascade(*a, *one->p, one->rows, DT, HD, a->gpw, one->prefix_wg,
                                             ygrid, st);
         if (e != hipSuccess) return e;
-      } else if (a->bs % 16 == 0 && staged)
-        hipLaunchKernelGGL((paged_decode_mfma_kernel<DT, GPW, true, HD, false, true>), grid, block, lds, st, *a);
-      else if (a->bs % 16 == 0)
-        hipLaunchKernelGGL((paged_decode_mfma_kernel<DT, GPW, true, HD, false>), grid, block, lds, st, *a);
-      else if (staged)
-        hipLaunchKernelGGL((paged_decode_mfma_kernel<DT, GPW, false, HD, false, true>), grid, block, lds, st, *a);
-      else
-        hipLaunchKernelGGL((paged_decode_mfma_kernel<DT, GPW, false, HD, false>), grid, block, lds, st, *a);
+      } else if (a->rows) {
+        launch_stream<DT, HD, GPW, true>(grid, block, lds, staged);
+      } else {
+        launch_stream<DT, HD, GPW, false>(grid, block, lds, staged);
+      }
     } else {
       hipLaunchKernelGGL((paged_decode_stream_kernel<DT, HD, GPW>), grid, block, 0, st, *a);
     }
@@ -158,11 +172,12 @@ struct LaunchDecode {
     if (e != hipSuccess || (a->num_wg <= 1 && !a->pre_row)) return e;
     if constexpr (use_mfma<DT, HD>()) {
       if (one) {  // after a one-launch cascade: its unit split
-        launch_combine<DT, HD, true>(*a, st);
+        launch_combine<DT, HD, true, false>(*a, st);
         return hipGetLastError();
       }
     }
-    launch_combine<DT, HD, false>(*a, st);
+    if (a->rows) launch_combine<DT, HD, false, true>(*a, st);
+    else launch_combine<DT, HD, false, false>(*a, st);
     return hipGetLastError();
   }
 };
@@ -360,11 +375,11 @@ int decode_ex(void* out, int out_dtype, int64_t out_stride_b, int64_t out_stride
               const float* prefix_out, const float* prefix_lse,
               const int32_t* prefix_row, int32_t prefix_parts,
               int64_t prefix_stride, void* stream,
-              const CascadeLaunch* one, bool check_only) {
+              const CascadeLaunch* one, bool check_only, const int64_t* rows, int64_t num_rows) {
   const int bad = check_decode_shape(kv_dtype, head_dim, num_heads, num_kv_heads);
   if (bad) return bad;
   const bool cascade = prefix_row != nullptr && prefix_parts > 0;
-  if (prefix_parts < 0 || prefix_stride < 0) return PKV_E_SHAPE;
+  if (prefix_parts < 0 || prefix_stride < 0 || num_rows < 0) return PKV_E_SHAPE;
   if (cascade && (!prefix_out || !prefix_lse)) return PKV_E_NULL;
   if (cascade && !aligned16(prefix_out)) return PKV_E_ALIGN;
   if (!(out_dtype == kv_dtype || out_dtype == PKV_F32)) return PKV_E_DTYPE;
@@ -442,6 +457,8 @@ int decode_ex(void* out, int out_dtype, int64_t out_stride_b, int64_t out_stride
   a.fin_lse = nullptr;
   a.fin_sb = a.fin_sh = 0;
   a.fin_f32 = 0;
+  a.rows = rows;
+  a.num_rows = num_rows;
   a.desc = nullptr;
   a.ws_acc = nullptr;
   a.ws_ml = nullptr;
@@ -574,6 +591,24 @@ int pkv_paged_decode(void* out, int out_dtype, int64_t out_stride_b, int64_t out
                              context_lens, batch, num_heads, num_kv_heads, head_dim, block_size,
                              scale, num_workgroups, workspace, workspace_bytes, nullptr,
                              nullptr, nullptr, nullptr, nullptr, 0, 0, stream);
+}
+
+int pkv_paged_decode_rows(void* out, int out_dtype, int64_t out_stride_b, int64_t out_stride_h,
+                          const void* q, int64_t q_stride_b, int64_t q_stride_h,
+                          const void* k_cache, const void* v_cache, int kv_dtype,
+                          int64_t kv_stride_slot, int64_t kv_stride_head, int64_t num_slots,
+                          const int32_t* block_tables, int64_t table_stride, int32_t max_blocks,
+                          const int32_t* context_lens, int32_t batch, int32_t num_heads,
+                          int32_t num_kv_heads, int32_t head_dim, int32_t block_size,
+                          float scale, int32_t num_workgroups, void* workspace,
+                          int64_t workspace_bytes, const int64_t* rows, int64_t num_rows,
+                          void* stream) {
+  return decode_ex(out, out_dtype, out_stride_b, out_stride_h, q, q_stride_b, q_stride_h, k_cache,
+                   v_cache, kv_dtype, kv_stride_slot, kv_stride_head, num_slots, block_tables,
+                   table_stride, max_blocks, context_lens, batch, num_heads, num_kv_heads,
+                   head_dim, block_size, scale, num_workgroups, workspace, workspace_bytes,
+                   nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0, stream, nullptr, false,
+                   rows, num_rows);
 }
 
 int pkv_paged_decode_ex(void* out, int out_dtype, int64_t out_stride_b, int64_t out_stride_h,

@@ -51,6 +51,10 @@ struct DecodeArgs {
   int64_t fin_sb, fin_sh;
   int fin_f32;
   float* fin_lse;
+  // Sequence b's row of q and out: rows[b] (null: b) of num_rows rows; negative values count
+  // from the end, and a sequence whose row lies outside writes nothing.
+  const int64_t* rows;
+  int64_t num_rows;
 };
 
 }  // namespace pkv
@@ -98,6 +102,15 @@ __device__ __forceinline__ int first_blk(const DecodeArgs& a, int b) {
   if (!a.first_block) return 0;
   const int f = a.first_block[b];
   return f < 0 ? 0 : (f > a.max_blocks ? a.max_blocks : f);
+}
+
+// Sequence b's row of q and out, or -1. The lookup is a memory trip of its own, but the
+// first K/V tiles do not wait for it.
+__device__ __forceinline__ int64_t seq_row(const DecodeArgs& a, int b) {
+  if (!a.rows) return b;
+  int64_t r = a.rows[b];
+  if (r < 0) r += a.num_rows;
+  return r >= 0 && r < a.num_rows ? r : -1;
 }
 
 // Where the stream pass writes a sequence it finishes whole: the result (out), except
@@ -367,10 +380,12 @@ paged_decode_stream_kernel(const DecodeArgs a) {
     ub = ue;
 
     // Query rows of this wave for sequence b, pre-scaled into the exp2 domain.
+    const int64_t srow = seq_row(a, b);
     float qf[GPW][VEC];
 #pragma unroll
     for (int g = 0; g < GPW; ++g) {
-      const S* qp = reinterpret_cast<const S*>(a.q) + b * a.q_sb + (int64_t)(h0 + g) * a.q_sh + d0;
+      const S* qp = reinterpret_cast<const S*>(a.q) + (srow < 0 ? 0 : srow) * a.q_sb +
+                    (int64_t)(h0 + g) * a.q_sh + d0;
       float t[VEC];
       unpack16<DT>(*reinterpret_cast<const uint4*>(qp), t);
 #pragma unroll
@@ -498,6 +513,7 @@ paged_decode_stream_kernel(const DecodeArgs a) {
 
     if (lane < LPT) {
       if (whole) {  // the whole context was in this range: final output directly
+        if (srow < 0) continue;
         const WholeDst dst = whole_dst(a, pre_b);
 #pragma unroll
         for (int g = 0; g < GPW; ++g) {
@@ -506,7 +522,7 @@ paged_decode_stream_kernel(const DecodeArgs a) {
           float o[VEC];
 #pragma unroll
           for (int c = 0; c < VEC; ++c) o[c] = acc[g][c] * inv;
-          const int64_t e = b * dst.sb + (int64_t)(h0 + g) * dst.sh + d0;
+          const int64_t e = srow * dst.sb + (int64_t)(h0 + g) * dst.sh + d0;
           if (dst.f32) store_vec<PKV_F32, VEC>((float*)dst.p + e, o);
           else store_vec<DT, VEC>((S*)dst.p + e, o);
           if (dst.lse && lane == 0) dst.lse[(int64_t)b * a.nh + h0 + g] = lse_of(m[g], l[g]);
@@ -561,6 +577,11 @@ template <int HD, int GPW, bool SPLIT = false> constexpr bool pv_mfma() {
   return GPW > 4 || (HD == 64 && !SPLIT && PKV_DECODE_PV_MFMA);
 }
 constexpr int kVSlotBytes = 4096;
+// The stream pass's instantiation for GPW heads per wave: with P.V on the matrix cores only
+// the wide one (its registers do not depend on the heads).
+template <int HD, int GPW> constexpr int stream_gpw() {
+  return pv_mfma<HD, GPW>() ? kWideHeads : GPW;
+}
 
 template <int DT> struct Mfma16x16x32;
 template <> struct Mfma16x16x32<PKV_BF16> {
@@ -701,7 +722,9 @@ __device__ __forceinline__ void split_merge(const DecodeArgs& a, int b, int h0,
     for (int k = 0; k < DPL; ++k) o[k] = __builtin_fmaf(wgt, part_acc[s][g][DPL * lane + k], o[k]);
   }
   const float inv = l > 0.f ? 1.f / l : 0.f;  // empty context: 0
-  const int64_t e = b * a.out_sb + (int64_t)(h0 + g) * a.out_sh + DPL * lane;
+  const int64_t srow = seq_row(a, b);
+  if (srow < 0) return;
+  const int64_t e = srow * a.out_sb + (int64_t)(h0 + g) * a.out_sh + DPL * lane;
 #pragma unroll
   for (int k = 0; k < DPL; ++k) {
     const float v = o[k] * inv;
@@ -724,6 +747,7 @@ __device__ __forceinline__ void split_merge_wide(const DecodeArgs& a, int b, int
   float* const part = reinterpret_cast<float*>(vslots);  // [wave][head of the round][HD]
   const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
   const int col = lane & 15, grp = lane >> 4;
+  const int64_t srow = seq_row(a, b);
   if (grp == 0 && col < ng) {
     part_ml[wave][col][0] = m_own;
     part_ml[wave][col][1] = l_own;
@@ -737,7 +761,7 @@ __device__ __forceinline__ void split_merge_wide(const DecodeArgs& a, int b, int
     }
     __syncthreads();
     const int g = g0 + wave;
-    if (g >= ng) continue;
+    if (g >= ng || srow < 0) continue;
     float mmax = -INFINITY;
 #pragma unroll
     for (int s = 0; s < W; ++s) mmax = fmaxf(mmax, part_ml[s][g][0]);
@@ -754,7 +778,7 @@ __device__ __forceinline__ void split_merge_wide(const DecodeArgs& a, int b, int
         o[k] = __builtin_fmaf(wgt, part[(s * W + wave) * HD + DPL * lane + k], o[k]);
     }
     const float inv = l > 0.f ? 1.f / l : 0.f;  // empty context: 0
-    const int64_t e = b * a.out_sb + (int64_t)(h0 + g) * a.out_sh + DPL * lane;
+    const int64_t e = srow * a.out_sb + (int64_t)(h0 + g) * a.out_sh + DPL * lane;
 #pragma unroll
     for (int k = 0; k < DPL; ++k) {
       const float v = o[k] * inv;
@@ -767,7 +791,9 @@ __device__ __forceinline__ void split_merge_wide(const DecodeArgs& a, int b, int
 // The MFMA stream pass of workgroup (bx, by): bx indexes the unit ranges (or, SPLIT, the
 // sequence), by the task group. vslots: kVSlotBytes of LDS per wave where P.V runs on the
 // matrix cores (pv_mfma), else unused.
-template <int DT, int GPW, bool FAST, int HD, bool SPLIT, bool STAGED = false, bool WT = false>
+// ROWS: a.rows may be non-null (always looked at in the split pass).
+template <int DT, int GPW, bool FAST, int HD, bool SPLIT, bool STAGED = false, bool WT = false,
+          bool ROWS = false>
 __device__ __forceinline__ void decode_mfma_body(const DecodeArgs& a, const int bx, const int by,
                                                  u32x4* const vslots) {
   static_assert(!WT || STAGED, "the one-launch cascade's split takes the staged pass");
@@ -897,7 +923,9 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeArgs& a, const int 
     // Q^T as the B operand: column col = query head h0 + col.
     u32x4 qb[4];
     {
-      const S* qp = reinterpret_cast<const S*>(a.q) + b * a.q_sb + (int64_t)(h0 + col) * a.q_sh + 8 * grp;
+      const int64_t srow = ROWS || SPLIT ? seq_row(a, b) : b;
+      const S* qp = reinterpret_cast<const S*>(a.q) + (srow < 0 ? 0 : srow) * a.q_sb +
+                    (int64_t)(h0 + col) * a.q_sh + 8 * grp;
 #pragma unroll
       for (int m = 0; m < KB; ++m)
         qb[m] = col < ng ? *reinterpret_cast<const u32x4*>(qp + 32 * m) : u32x4{0, 0, 0, 0};
@@ -1337,7 +1365,11 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeArgs& a, const int 
         if (whole) {
           const WholeDst dst = whole_dst(a, pre_b);
           const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
-          const int64_t e = b * dst.sb + (int64_t)(h0 + col) * dst.sh + 4 * grp;
+          const int64_t srow = ROWS ? seq_row(a, b) : b;
+          if constexpr (ROWS) {
+            if (srow < 0) continue;
+          }
+          const int64_t e = srow * dst.sb + (int64_t)(h0 + col) * dst.sh + 4 * grp;
 #pragma unroll
           for (int d = 0; d < NOV; ++d) {
             const f32x4 o4 = ov[d] * kOScale * inv;
@@ -1378,13 +1410,17 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeArgs& a, const int 
       const int d0 = 8 * col;
       if (whole) {
         const WholeDst dst = whole_dst(a, pre_b);
+        const int64_t srow = ROWS ? seq_row(a, b) : b;
+        if constexpr (ROWS) {
+          if (srow < 0) continue;
+        }
 #pragma unroll
         for (int g = 0; g < GPW; ++g) {
           const float inv = lh[g] > 0.f ? 1.f / lh[g] : 0.f;
           float o[8];
 #pragma unroll
           for (int d = 0; d < 8; ++d) o[d] = acc[g][d] * inv;
-          const int64_t e = b * dst.sb + (int64_t)(h0 + g) * dst.sh + d0;
+          const int64_t e = srow * dst.sb + (int64_t)(h0 + g) * dst.sh + d0;
           if (dst.f32) store_vec<PKV_F32, 8>((float*)dst.p + e, o);
           else store_vec<DT, 8>((S*)dst.p + e, o);
           if (dst.lse && col == 0) dst.lse[(int64_t)b * a.nh + h0 + g] = lse_of(mh[g], lh[g]);
@@ -1403,12 +1439,12 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeArgs& a, const int 
 }
 
 // Dynamic LDS: kVSlotBytes per wave where P.V runs on the matrix cores (pv_mfma).
-template <int DT, int GPW, bool FAST, int HD, bool SPLIT, bool STAGED = false>
+template <int DT, int GPW, bool FAST, int HD, bool SPLIT, bool STAGED = false, bool ROWS = false>
 __global__ void __launch_bounds__(512)
 paged_decode_mfma_kernel(const DecodeArgs a) {
   extern __shared__ __align__(16) u32x4 decode_vslots[];
-  decode_mfma_body<DT, GPW, FAST, HD, SPLIT, STAGED>(a, (int)blockIdx.x, (int)blockIdx.y,
-                                                     decode_vslots);
+  decode_mfma_body<DT, GPW, FAST, HD, SPLIT, STAGED, false, ROWS>(a, (int)blockIdx.x,
+                                                                 (int)blockIdx.y, decode_vslots);
 }
 
 // ---------------------------------------------------------------------------------
@@ -1455,7 +1491,7 @@ __device__ void seq_units(const DecodeArgs& a, int b, int64_t* ub, int64_t* ue, 
 // SP = 1: one wave per (sequence, query head). SP > 1 (batches with few such pairs): SP
 // waves per pair, each folding its share of the records, their states merged through
 // LDS -- 1 / SP of the dependent round trips for a sequence cut into many pieces.
-template <int DT, int HD, int SP, bool WT = false>
+template <int DT, int HD, int SP, bool WT = false, bool ROWS = false>
 __global__ void __launch_bounds__(SP > 4 ? SP * kWave : 256)
 paged_decode_combine_kernel(const DecodeArgs a) {
   static_assert(SP == 1 || SP == 2 || SP == 4 || SP == 8 || SP == 16, "waves per (sequence, head)");
@@ -1477,6 +1513,7 @@ paged_decode_combine_kernel(const DecodeArgs a) {
   const int b = pw / a.nh, h = pw - b * a.nh;
 
   const int4 plan = a.desc[b];
+  const int64_t srow = ROWS ? seq_row(a, b) : b;  // fetched with the plan
   const bool cascade = a.pre_row != nullptr;
   const int pre_b = cascade ? a.pre_row[b] : -1;  // fetched with the plan
   const int pre = part == 0 ? pre_b : -1;
@@ -1619,6 +1656,9 @@ paged_decode_combine_kernel(const DecodeArgs a) {
       parts.fold(mmax, lsum, out_acc);
     }
   }
+  if constexpr (ROWS) {
+    if (srow < 0) return;
+  }
   const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
   float* lse_dst = cascade ? a.fin_lse : a.lse;
   if (lse_dst && lane == 0) lse_dst[(int64_t)b * a.nh + h] = lse_of(mmax, lsum);
@@ -1630,7 +1670,7 @@ paged_decode_combine_kernel(const DecodeArgs a) {
     const int d = lane + kWave * k;
     if (d >= HD) break;
     const float o = out_acc[k] * inv;
-    const int64_t e = b * sb + (int64_t)h * sh + d;
+    const int64_t e = srow * sb + (int64_t)h * sh + d;
     if (f32) reinterpret_cast<float*>(dst)[e] = o;
     else reinterpret_cast<typename Elt<DT>::S*>(dst)[e] = Elt<DT>::from_f32(o);
   }

@@ -74,9 +74,10 @@ paged_prefill_rows_kernel(const PrefillArgs a) {
     const int p = e / HD, d = e - p * HD;
     const int i = tok0 + p / GPW, h = h0 + p % GPW;
     float x = 0.f;
-    const int row = i < ql ? (a.q_rows ? a.q_rows[q0 + i] : q0 + i) : -1;
+    int64_t row = -1;
+    if (i < ql) row = a.rows ? token_row(a, q0 + i) : a.q_rows ? a.q_rows[q0 + i] : q0 + i;
     if (row >= 0 && h < hend)  // a negative q_rows entry: no query there
-      x = Elt<DT>::to_f32(reinterpret_cast<const S*>(a.q)[(int64_t)row * a.q_st +
+      x = Elt<DT>::to_f32(reinterpret_cast<const S*>(a.q)[row * a.q_st +
                                                         (int64_t)h * a.q_sh + d]);
     qs[wave][p][d] = x * a.scale_log2;
   }
@@ -188,11 +189,13 @@ paged_prefill_rows_kernel(const PrefillArgs a) {
     if (i >= ql || h >= hend || (a.q_rows && a.q_rows[q0 + i] < 0)) continue;
     const float inv = lt > 0.f ? 1.f / lt : 0.f;  // nothing visible: 0
     const int64_t t = q0 + i;
+    const int64_t orow = a.rows ? token_row(a, t) : t;
+    if (orow < 0) continue;
 #pragma unroll
     for (int k = 0; k < DPL; ++k) {
       const int d = lane + kWave * k;
       if (d >= HD) break;
-      const int64_t e = t * a.out_st + (int64_t)h * a.out_sh + d;
+      const int64_t e = orow * a.out_st + (int64_t)h * a.out_sh + d;
       const float o = acc[p][k] * inv;
       if (a.out_f32) reinterpret_cast<float*>(a.out)[e] = o;
       else reinterpret_cast<S*>(a.out)[e] = Elt<DT>::from_f32(o);
@@ -205,7 +208,7 @@ paged_prefill_rows_kernel(const PrefillArgs a) {
 // Host-side dispatch.
 // ---------------------------------------------------------------------------------
 
-template <int DT, int HD>
+template <int DT, int HD, bool ROWS>
 hipError_t launch_prefill_hd(PrefillArgs a, int64_t rows, hipStream_t st) {
   constexpr int BM = PrefillShape<HD>::BM;
   a.row_blocks = (int)((rows + BM - 1) / BM);
@@ -215,26 +218,26 @@ hipError_t launch_prefill_hd(PrefillArgs a, int64_t rows, hipStream_t st) {
   if constexpr (DT == PKV_BF16) {
     if (a.v16) {  // P.V in fp16 against the copy of V
       if (a.bs_shift >= 0)
-        hipLaunchKernelGGL((paged_prefill_kernel<DT, HD, true, true>), grid, block, 0, st, a);
+        hipLaunchKernelGGL((paged_prefill_kernel<DT, HD, true, true, ROWS>), grid, block, 0, st, a);
       else
-        hipLaunchKernelGGL((paged_prefill_kernel<DT, HD, false, true>), grid, block, 0, st, a);
+        hipLaunchKernelGGL((paged_prefill_kernel<DT, HD, false, true, ROWS>), grid, block, 0, st, a);
       return hipGetLastError();
     }
   }
   if (a.bs_shift >= 0)
-    hipLaunchKernelGGL((paged_prefill_kernel<DT, HD, true, false>), grid, block, 0, st, a);
+    hipLaunchKernelGGL((paged_prefill_kernel<DT, HD, true, false, ROWS>), grid, block, 0, st, a);
   else
-    hipLaunchKernelGGL((paged_prefill_kernel<DT, HD, false, false>), grid, block, 0, st, a);
+    hipLaunchKernelGGL((paged_prefill_kernel<DT, HD, false, false, ROWS>), grid, block, 0, st, a);
   return hipGetLastError();
 }
 
-template <int DT>
+template <int DT, bool ROWS>
 hipError_t launch_prefill(const PrefillArgs& a, int hd, int64_t rows, hipStream_t st) {
   switch (hd) {
-    case 32: return launch_prefill_hd<DT, 32>(a, rows, st);
-    case 64: return launch_prefill_hd<DT, 64>(a, rows, st);
-    case 128: return launch_prefill_hd<DT, 128>(a, rows, st);
-    default: return launch_prefill_hd<DT, 256>(a, rows, st);
+    case 32: return launch_prefill_hd<DT, 32, ROWS>(a, rows, st);
+    case 64: return launch_prefill_hd<DT, 64, ROWS>(a, rows, st);
+    case 128: return launch_prefill_hd<DT, 128, ROWS>(a, rows, st);
+    default: return launch_prefill_hd<DT, 256, ROWS>(a, rows, st);
   }
 }
 
@@ -353,6 +356,8 @@ int prefill_args(PrefillArgs* out_args, int64_t* rows_out, void* out, int out_dt
   a.v16 = nullptr;
   a.v16_k = nullptr;
   a.v16_kstride = 0;
+  a.rows = nullptr;
+  a.rows_len = a.num_rows = 0;
   return 0;
 }
 
@@ -369,12 +374,15 @@ int run_prefill(const PrefillArgs& a, int64_t rows, int kv_dtype, int head_dim,
     return (int)(kv_dtype == PKV_BF16 ? launch_rows<PKV_BF16>(a, head_dim, max_query_len, st)
                                       : launch_rows<PKV_F16>(a, head_dim, max_query_len, st));
   }
-  if (kv_dtype == PKV_F16) return (int)launch_prefill<PKV_F16>(a, head_dim, rows, st);
+  if (kv_dtype == PKV_F16)
+    return (int)(a.rows ? launch_prefill<PKV_F16, true>(a, head_dim, rows, st)
+                        : launch_prefill<PKV_F16, false>(a, head_dim, rows, st));
   if (a.v16) {
     const hipError_t e = launch_v16(a, head_dim, st);
     if (e != hipSuccess) return (int)e;
   }
-  return (int)launch_prefill<PKV_BF16>(a, head_dim, rows, st);
+  return (int)(a.rows ? launch_prefill<PKV_BF16, true>(a, head_dim, rows, st)
+                      : launch_prefill<PKV_BF16, false>(a, head_dim, rows, st));
 }
 
 // Whether a call of these shapes can use the fp16 V copy: bf16 at head_dim 32..256,
@@ -462,15 +470,40 @@ int pkv_paged_prefill_ws(void* out, int out_dtype, int64_t out_stride_tok, int64
                          int32_t n_chunks, int32_t max_query_len, int32_t num_heads,
                          int32_t num_kv_heads, int32_t head_dim, int32_t block_size, float scale,
                          void* workspace, int64_t workspace_bytes, void* stream) {
+  return pkv_paged_prefill_rows(out, out_dtype, out_stride_tok, out_stride_h, q, q_stride_tok,
+                                q_stride_h, k_cache, v_cache, kv_dtype, kv_stride_slot,
+                                kv_stride_head, num_slots, block_tables, table_stride, max_blocks,
+                                context_lens, cu_seqlens_q, n_chunks, max_query_len, num_heads,
+                                num_kv_heads, head_dim, block_size, scale, workspace,
+                                workspace_bytes, nullptr, 0, 0, stream);
+}
+
+int pkv_paged_prefill_rows(void* out, int out_dtype, int64_t out_stride_tok, int64_t out_stride_h,
+                           const void* q, int64_t q_stride_tok, int64_t q_stride_h,
+                           const void* k_cache, const void* v_cache, int kv_dtype,
+                           int64_t kv_stride_slot, int64_t kv_stride_head, int64_t num_slots,
+                           const int32_t* block_tables, int64_t table_stride, int32_t max_blocks,
+                           const int32_t* context_lens, const int32_t* cu_seqlens_q,
+                           int32_t n_chunks, int32_t max_query_len, int32_t num_heads,
+                           int32_t num_kv_heads, int32_t head_dim, int32_t block_size,
+                           float scale, void* workspace, int64_t workspace_bytes,
+                           const int64_t* rows, int64_t rows_len, int64_t num_rows,
+                           void* stream) {
+  if (rows_len < 0 || num_rows < 0 || num_rows > 0x7FFFFFFF) return PKV_E_SHAPE;
   PrefillArgs a;
-  int64_t rows = 0;
-  const int bad = prefill_args(&a, &rows, out, out_dtype, out_stride_tok, out_stride_h, q,
+  int64_t qrows = 0;  // query rows of the longest chunk for one KV head
+  const int bad = prefill_args(&a, &qrows, out, out_dtype, out_stride_tok, out_stride_h, q,
                                q_stride_tok, q_stride_h, k_cache, v_cache, kv_dtype,
                                kv_stride_slot, kv_stride_head, num_slots, block_tables,
                                table_stride, max_blocks, context_lens, cu_seqlens_q, n_chunks,
                                max_query_len, num_heads, num_kv_heads, head_dim, block_size,
                                scale, 1, nullptr, nullptr);
   if (bad) return bad == 1 ? 0 : bad;
+  if (rows) {
+    a.rows = rows;
+    a.rows_len = rows_len;
+    a.num_rows = num_rows;
+  }
   if (workspace_bytes < 0 || (workspace_bytes > 0 && !workspace)) return PKV_E_WORKSPACE;
   if (workspace && !aligned16(workspace)) return PKV_E_ALIGN;
   if (workspace && v16_shapes(kv_dtype, head_dim, max_blocks, block_size, num_slots)) {
@@ -481,7 +514,7 @@ int pkv_paged_prefill_ws(void* out, int out_dtype, int64_t out_stride_tok, int64
       a.v16 = static_cast<const char*>(workspace) + l.k_bytes;
     }
   }
-  return run_prefill(a, rows, kv_dtype, head_dim, max_query_len, (hipStream_t)stream);
+  return run_prefill(a, qrows, kv_dtype, head_dim, max_query_len, (hipStream_t)stream);
 }
 
 }  // extern "C"

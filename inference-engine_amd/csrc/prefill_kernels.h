@@ -41,7 +41,19 @@ struct PrefillArgs {
   const void* v16;
   const uint8_t* v16_k;
   int32_t v16_kstride;
+  // Query token t's row of q and out: rows[t], t < rows_len (null: t), of num_rows rows;
+  // negative values count from the end, a row outside is skipped. Not with q_rows.
+  const int64_t* rows;
+  int64_t rows_len, num_rows;
 };
+
+// Query token t's row of q and out through `rows` (non-null), or -1.
+__device__ __forceinline__ int64_t token_row(const PrefillArgs& a, int64_t t) {
+  if (t >= a.rows_len) return -1;
+  int64_t r = a.rows[t];
+  if (r < 0) r += a.num_rows;
+  return r >= 0 && r < a.num_rows ? r : -1;
+}
 
 // Tokens per region tile of the fp16 V copy (one workgroup of the copy kernel, one scale
 // exponent); regions are padded to a multiple of it.
@@ -350,7 +362,8 @@ template <int HD> struct PrefillLds {
 // copy. Every exit is workgroup-uniform except half 1's after the merge; a caller that
 // runs several items on one workgroup puts a barrier between them (the merge reuses the
 // rings).
-template <int DT, int HD, bool POW2, bool V16>
+// ROWS: q and out rows through a.rows (else a.rows is null).
+template <int DT, int HD, bool POW2, bool V16, bool ROWS>
 __device__ __forceinline__ void prefill_body(const PrefillArgs& a, const PrefillItem& it,
                                              PrefillLds<HD>& lds) {
   using SH = PrefillShape<HD>;
@@ -381,6 +394,7 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs& a, const Prefill
   // This lane's query row in each of its wave's 16-row tiles (B operand column). Both
   // halves hold the same rows.
   int row_tok[RT];
+  int row_out[RT];  // the row of out
   bool row_ok[RT];
   u32x4 qf[RT][KS];
 #pragma unroll
@@ -390,7 +404,12 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs& a, const Prefill
     const int rr = row_ok[t] ? rho : 0;
     row_tok[t] = rr / G;
     int64_t qrow = q0 + row_tok[t];
-    if (a.q_rows) {  // a negative entry: no query there (nothing read or written)
+    if constexpr (ROWS) {
+      const int64_t r = token_row(a, qrow);
+      row_ok[t] = row_ok[t] && r >= 0;
+      qrow = r >= 0 ? r : 0;
+      row_out[t] = (int)qrow;
+    } else if (a.q_rows) {  // a negative entry: no query there (nothing read or written)
       const int qr = a.q_rows[q0 + row_tok[t]];
       row_ok[t] = row_ok[t] && qr >= 0;
       qrow = qr >= 0 ? qr : 0;
@@ -1073,7 +1092,7 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs& a, const Prefill
     if (a.lse && grp == 0)  // log2 normaliser: the exponent reference m_run plus log2(sum)
       a.lse[(int64_t)(q0 + rho / G) * a.nh + kvh * G + rho % G] =
           l_tot > 0.f ? m_run[t] + (__log2f(l_tot) - PM::kPLog2) : -INFINITY;
-    const int64_t e0 = (int64_t)(q0 + rho / G) * a.out_st + (int64_t)(kvh * G + rho % G) * a.out_sh;
+    const int64_t e0 = (ROWS ? (int64_t)row_out[t] : (int64_t)(q0 + rho / G)) * a.out_st + (int64_t)(kvh * G + rho % G) * a.out_sh;
 #pragma unroll
     for (int d = 0; d < DTL; ++d) {
       const int64_t e = e0 + 16 * d + 4 * grp;
@@ -1093,7 +1112,7 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs& a, const Prefill
 // exit is workgroup-uniform except half 1's after the merge; a caller that runs several
 // items on one workgroup puts a barrier between them (the merge reuses the rings).
 // V16: V from the fp16 copy (bf16 caches; the launch guarantees every chunk's region).
-template <int DT, int HD, bool POW2, bool V16 = false>
+template <int DT, int HD, bool POW2, bool V16, bool ROWS>
 __device__ __forceinline__ void prefill_item(const PrefillArgs& a, const int item,
                                              PrefillLds<HD>& lds) {
   const int lane = threadIdx.x & (kWave - 1);
@@ -1128,7 +1147,7 @@ __device__ __forceinline__ void prefill_item(const PrefillArgs& a, const int ite
     it.q1 = a.cu_q[it.c + 1];
     it.n = min(max(a.ctx[it.c], 0), cap);
   }
-  prefill_body<DT, HD, POW2, V16>(a, it, lds);
+  prefill_body<DT, HD, POW2, V16, ROWS>(a, it, lds);
 }
 
 // Head_dim 32 and 64 leave room for two workgroups on a CU (72 KB of LDS each at 64): the
@@ -1140,11 +1159,11 @@ template <int DT, int HD, bool V16> constexpr bool prefill_two_wgs() {
   return HD <= 64 && (DT != PKV_BF16 || V16);
 }
 
-template <int DT, int HD, bool POW2, bool V16>
+template <int DT, int HD, bool POW2, bool V16, bool ROWS>
 __global__ void __launch_bounds__(512, (prefill_two_wgs<DT, HD, V16>()) ? 4 : 2)
 paged_prefill_kernel(const PrefillArgs a) {
   __shared__ __align__(16) PrefillLds<HD> lds;
-  prefill_item<DT, HD, POW2, V16>(a, (int)blockIdx.x, lds);
+  prefill_item<DT, HD, POW2, V16, ROWS>(a, (int)blockIdx.x, lds);
 }
 
 // The fp16 copy of the chunks' V for the bf16 matrix-core prefill (PrefillArgs::v16):

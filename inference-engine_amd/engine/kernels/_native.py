@@ -18,7 +18,7 @@ LIB_PATH = os.path.join(
     "lib",
     "libpaged_kv.so",
 )
-ABI_VERSION = 5
+ABI_VERSION = 6
 PKV_NOALLOC_SCRATCH_BYTES = 32 << 20  # include/paged_kv.h
 
 PKV_F32, PKV_F16, PKV_BF16 = 0, 1, 2
@@ -57,6 +57,16 @@ SIGNATURES: dict[str, tuple] = {
          _p, _i64, _i32,                          # block tables
          _p, _i32, _i32, _i32, _i32, _i32,        # ctx, batch, nh, nkv, hd, bs
          _f32, _i32, _p],                         # scale, wgs, stream
+    ),  # fmt: skip
+    "pkv_paged_decode_rows": (
+        ctypes.c_int,
+        [_p, ctypes.c_int, _i64, _i64,            # out
+         _p, _i64, _i64,                          # q
+         _p, _p, ctypes.c_int, _i64, _i64, _i64,  # k, v caches
+         _p, _i64, _i32,                          # block tables
+         _p, _i32, _i32, _i32, _i32, _i32,        # ctx, batch, nh, nkv, hd, bs
+         _f32, _i32, _p, _i64,                    # scale, wgs, workspace
+         _p, _i64, _p],                           # rows, num_rows, stream
     ),  # fmt: skip
     "pkv_rms_norm": (
         ctypes.c_int,
@@ -120,6 +130,16 @@ SIGNATURES: dict[str, tuple] = {
          _p, _p, _i32, _i32,                      # ctx, cu_q, n_chunks, max_query_len
          _i32, _i32, _i32, _i32, _f32,            # nh, nkv, hd, bs, scale
          _p, _i64, _p],                           # workspace, bytes, stream
+    ),  # fmt: skip
+    "pkv_paged_prefill_rows": (
+        ctypes.c_int,
+        [_p, ctypes.c_int, _i64, _i64,            # out
+         _p, _i64, _i64,                          # q
+         _p, _p, ctypes.c_int, _i64, _i64, _i64,  # k, v caches
+         _p, _i64, _i32,                          # block tables
+         _p, _p, _i32, _i32,                      # ctx, cu_q, n_chunks, max_query_len
+         _i32, _i32, _i32, _i32, _f32,            # nh, nkv, hd, bs, scale
+         _p, _i64, _p, _i64, _i64, _p],           # workspace, bytes, rows, len, num_rows, stream
     ),  # fmt: skip
 }
 

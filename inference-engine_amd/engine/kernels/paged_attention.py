@@ -348,6 +348,7 @@ def paged_decode_attention(
     workspace: torch.Tensor | None = None,
     prefix_groups: PrefixGroups | None = None,
     prefix_workgroups: int | None = None,
+    rows: torch.Tensor | None = None,
 ) -> torch.Tensor:
     """q: [B, nh, hd]; k_cache, v_cache: [num_slots, nkv, hd] (one layer);
     block_tables: [B, max_blocks] int32; context_lens: [B] int32 -> [B, nh, hd].
@@ -370,15 +371,26 @@ def paged_decode_attention(
     prefix pass and the decode pass share one launch: ``prefix_workgroups`` of the
     workgroups (None: the library's default) take the prefix items while the others
     stream the private blocks; a negative value runs them as two launches.
+    ``rows`` (int64 [B], with ``out``): q and out hold one row per token of a larger step, and
+    sequence b's are row ``rows[b]`` of both -- ``out[rows] = attention(q[rows])`` without the
+    gather and the scatter (``rows_in_place`` says whether their layouts allow it; not with
+    ``prefix_groups``). Rows that no sequence names keep what they hold.
     """
     del block_n
     what = "paged_decode_attention"
-    dev = _check_decode_args(what, q, k_cache, v_cache, block_tables, context_lens, block_size)
-    b, nh, hd = q.shape
+    dev = _check_decode_args(what, q, k_cache, v_cache, block_tables, context_lens, block_size,
+                             rows)  # fmt: skip
+    b = q.shape[0] if rows is None else rows.numel()
+    _, nh, hd = q.shape
     nkv = k_cache.shape[1]
     kv_code = _native.dtype_code(k_cache.dtype, what)
 
-    q = q.contiguous()
+    if rows is None:
+        q = q.contiguous()
+    else:
+        _check_rows(what, q, out, rows)
+        if prefix_groups is not None:
+            raise ValueError(f"{what}: rows and prefix_groups do not go together")
     if out is None:
         out = torch.empty_like(q)
     else:
@@ -431,6 +443,9 @@ def paged_decode_attention(
             pg.q_rows.data_ptr(), o_pre.data_ptr(), lse_pre.data_ptr(),
             pg.prefix_row.data_ptr(), pg.pieces, pg.members, pwg, _native.stream_of(dev),
         )  # fmt: skip
+    elif rows is not None:
+        status = lib.pkv_paged_decode_rows(*common, rows.data_ptr(), q.shape[0],
+                                           _native.stream_of(dev))  # fmt: skip
     else:
         status = lib.pkv_paged_decode_ex(*common, None, None, None, None, None, 0, 0,
                                          _native.stream_of(dev))  # fmt: skip
@@ -486,13 +501,46 @@ def _check_out(what: str, out: torch.Tensor, q: torch.Tensor, dev: torch.device)
         raise ValueError(f"{what}: out must be [B, nh, hd] of {q.dtype} or float32 on {dev}")
 
 
+def rows_in_place(q: torch.Tensor, out: torch.Tensor, rows: torch.Tensor) -> bool:
+    """Whether the kernels can read rows of ``q`` and write rows of ``out`` in place
+    (``rows=``): [N, nh, hd] tensors of one dtype, unit stride in hd, 16-byte aligned rows and
+    heads that do not overlap (token- or head-major), apart in memory or the same tensor (a
+    query row is read before its result is written, by the same waves); ``rows`` a contiguous
+    int64 vector."""
+    if rows.dtype != torch.int64 or rows.dim() != 1 or not rows.is_contiguous() or \
+            rows.device != q.device or q.dim() != 3 or out.shape != q.shape or \
+            out.dtype != q.dtype or out.device != q.device:  # fmt: skip
+        return False
+    n, nh, hd = q.shape
+    size = q.element_size()
+    ends = []
+    for x in (q, out):
+        s0, s1, s2 = x.stride()
+        if s2 != 1 or s0 * size % 16 or s1 * size % 16 or x.data_ptr() % 16 or \
+                not (s1 >= hd and s0 >= (nh - 1) * s1 + hd or
+                     s0 >= hd and s1 >= (n - 1) * s0 + hd):  # fmt: skip
+            return False
+        ends.append(x.data_ptr() + ((n - 1) * s0 + (nh - 1) * s1 + hd) * size)
+    return n == 0 or (q.data_ptr() == out.data_ptr() and q.stride() == out.stride()) or \
+        ends[0] <= out.data_ptr() or ends[1] <= q.data_ptr()  # fmt: skip
+
+
+def _check_rows(what: str, q: torch.Tensor, out: torch.Tensor | None, rows: torch.Tensor) -> None:
+    if out is None or not rows_in_place(q, out, rows):
+        raise ValueError(f"{what}: rows needs out, with layouts that rows_in_place takes")
+    if _native.debug_checks() and bool(((rows < -q.shape[0]) | (rows >= q.shape[0])).any()):
+        raise IndexError(f"{what}: rows outside the {q.shape[0]} rows of q")
+
+
 def _check_decode_args(what, q, k_cache, v_cache, block_tables, context_lens,
-                       block_size) -> torch.device:  # fmt: skip
+                       block_size, rows=None) -> torch.device:  # fmt: skip
     """The decode entry points' argument checks (before any launch); returns the device."""
     dev = _native.require_gpu(what, q, k_cache, v_cache, block_tables, context_lens)
     if q.dim() != 3 or k_cache.dim() != 3 or v_cache.dim() != 3:
         raise ValueError(f"{what}: q, k_cache, v_cache must be 3-D")
     b, nh, hd = q.shape
+    if rows is not None:
+        b = rows.numel()
     nkv = k_cache.shape[1]
     if v_cache.shape != k_cache.shape or k_cache.shape[2] != hd:
         raise ValueError(f"{what}: cache shapes {tuple(k_cache.shape)}, "
@@ -578,6 +626,7 @@ def paged_prefill_attention(
     *,
     out: torch.Tensor | None = None,
     workspace: torch.Tensor | None = None,
+    rows: torch.Tensor | None = None,
 ) -> torch.Tensor:
     """Bottom-right causal attention of prompt chunks over the paged pool.
 
@@ -600,7 +649,8 @@ def paged_prefill_attention(
     hi + lo pair; ``workspace`` (a CUDA byte tensor of at least
     ``prefill_workspace_bytes(...)``) supplies it, else the call allocates one of that
     size through torch (at most ``PREFILL_WORKSPACE_MAX_BYTES``; beyond it, and for other
-    dtypes, the call takes no copy).
+    dtypes, the call takes no copy). ``rows`` (int64 [T], with ``out``): token t's query is row
+    ``rows[t]`` of q and its result goes to that row of out, as in ``paged_decode_attention``.
     """
     what = "paged_prefill_attention"
     dev = _native.require_gpu(what, q, k_cache, v_cache, block_tables, context_lens,
@@ -626,7 +676,11 @@ def paged_prefill_attention(
     if block_tables.dim() != 2 or block_tables.shape[0] != n_chunks or \
             block_tables.stride(1) != 1 or cu_seqlens_q.shape != (n_chunks + 1,):  # fmt: skip
         raise ValueError(f"{what}: block_tables [C, W], context_lens [C], cu_seqlens_q [C+1]")
-    q = q.contiguous()
+    if rows is None:
+        q = q.contiguous()
+    else:
+        _check_rows(what, q, out, rows)
+        t = rows.numel()
     if out is None:
         out = torch.empty_like(q)
     elif out.shape != q.shape or out.dtype not in (q.dtype, torch.float32) or \
@@ -651,14 +705,16 @@ def paged_prefill_attention(
         raise ValueError(f"{what}: workspace must be a contiguous tensor on {dev}")
     ws_ptr = workspace.data_ptr() if workspace is not None else None
     ws_bytes = workspace.numel() * workspace.element_size() if workspace is not None else 0
-    status = _native.lib().pkv_paged_prefill_ws(
+    status = _native.lib().pkv_paged_prefill_rows(
         out.data_ptr(), _native.dtype_code(out.dtype, what), out.stride(0), out.stride(1),
         q.data_ptr(), q.stride(0), q.stride(1),
         k_cache.data_ptr(), v_cache.data_ptr(), kv_code,
         k_cache.stride(0), k_cache.stride(1), k_cache.shape[0],
         block_tables.data_ptr(), block_tables.stride(0), block_tables.shape[1],
         context_lens.data_ptr(), cu_seqlens_q.data_ptr(), n_chunks, int(max_query_len),
-        nh, nkv, hd, block_size, hd**-0.5, ws_ptr, ws_bytes, _native.stream_of(dev),
+        nh, nkv, hd, block_size, hd**-0.5, ws_ptr, ws_bytes,
+        None if rows is None else rows.data_ptr(), 0 if rows is None else t,
+        0 if rows is None else q.shape[0], _native.stream_of(dev),
     )  # fmt: skip
     _native.check(status, what)
     return out

@@ -14,7 +14,11 @@ from __future__ import annotations
 
 import torch
 
-from engine.kernels.paged_attention import paged_decode_attention, paged_prefill_attention
+from engine.kernels.paged_attention import (
+    paged_decode_attention,
+    paged_prefill_attention,
+    rows_in_place,
+)
 from engine.runtime.paged_cache import PagedBatch
 
 
@@ -57,11 +61,20 @@ def mixed_attention(layer_idx: int, q: torch.Tensor, batch: PagedBatch,
     kc, vc, bs = cache.k[layer_idx], cache.v[layer_idx], cache.block_size
     if out is None:
         out = torch.empty_like(q)
-    if batch.block_tables is not None:
+    # The kernels take their rows of q and out through the index itself; layouts they cannot
+    # address go through gathered copies.
+    if batch.block_tables is not None and rows_in_place(q, out, batch.decode_rows):
+        paged_decode_attention(q, kc, vc, batch.block_tables, batch.context_lens, bs, out=out,
+                               rows=batch.decode_rows)  # fmt: skip
+    elif batch.block_tables is not None:
         rows = batch.decode_rows
         out[rows] = paged_decode_attention(q[rows], kc, vc, batch.block_tables,
                                            batch.context_lens, bs).to(out.dtype)  # fmt: skip
-    if batch.chunk_rows is not None:
+    if batch.chunk_rows is not None and rows_in_place(q, out, batch.chunk_rows):
+        paged_prefill_attention(q, kc, vc, batch.chunk_tables, batch.chunk_ctx, bs,
+                                batch.cu_seqlens_q, batch.max_query_len, out=out,
+                                rows=batch.chunk_rows)  # fmt: skip
+    elif batch.chunk_rows is not None:
         rows = batch.chunk_rows
         out[rows] = paged_prefill_attention(q[rows], kc, vc, batch.chunk_tables,
                                             batch.chunk_ctx, bs, batch.cu_seqlens_q,
