@@ -1,6 +1,7 @@
 // prefill.hip -- chunked-prefill attention (include/paged_kv.h: pkv_paged_prefill*): the
 // argument checks and launches of the matrix-core kernel (prefill_kernels.h, also
-// cascade decode's prefix pass), and the VALU kernel for fp32 K/V and head_dim 16.
+// cascade decode's prefix pass), and the fp32 matrix-core kernel for fp32 K/V and
+// head_dim 16.
 
 #include "cascade.h"
 #include "prefill_kernels.h"
@@ -10,198 +11,236 @@ namespace {
 using namespace pkv;
 
 // ---------------------------------------------------------------------------------
-// Chunked-prefill attention on the VALU, for the shapes the matrix-core kernel does not
-// take: fp32 K/V (any supported head_dim) and 16-bit K/V at head_dim 16. Same contract
-// and arguments as paged_prefill_kernel (causal / non-causal, q_rows, lse).
+// Chunked-prefill attention in fp32 arithmetic, for the shapes the 16-bit matrix-core kernel
+// does not take: fp32 K/V (any supported head_dim) and 16-bit K/V at head_dim 16 (widened as
+// they are staged). Same contract and arguments as paged_prefill_kernel (causal /
+// non-causal, q_rows, rows, lse); keys whose slot lies outside the pool are left out.
 //
-// A workgroup of 4 waves takes 16 consecutive query tokens of one chunk and GPW query
-// heads of one KV head; wave w holds tokens 4w .. 4w + 3, so P = 4 * GPW (token, head)
-// pairs per wave. Per tile of TK keys the workgroup stages K and V (converted to fp32)
-// and a liveness flag per key in LDS once, so every K/V row is read once per 16 query
-// tokens rather than once per token. Then, per wave:
-//   * scores with lane j = key j (TK = 32 at head_dim 256: lanes j and j + 32 split the
-//     head dims), the pairs' pre-scaled queries read from LDS as broadcast float4s;
-//   * fp32 online softmax per pair (tile max across lanes; each lane keeps its own share
-//     of the running sum), the probabilities of the tile written to LDS;
-//   * P.V with lane = head dim, the probabilities read back four keys at a time.
+// A workgroup of 8 waves takes 64 query rows (token, head of one KV head's group), so every
+// K/V tile it stages serves 64 of them, and two halves of its waves take the two halves of
+// the key tiles; wave w of a half holds rows 16 w .. 16 w + 15. Per tile of TK keys:
+//   * S^T = K . Q^T with v_mfma_f32_16x16x4_f32 (fp32 products and sums). The four k-slots of
+//     MFMA j of a 16-dim step are dims 16 i + 4 grp + j for lane group grp, so a lane reads
+//     its K operands as one 16-byte row piece and holds Q in registers the same way. Lane
+//     (row col, grp) gets keys 16 beta + 4 grp + r of query row col.
+//   * fp32 online softmax per row in that layout.
+//   * O^T += V^T . P^T with k-slot grp = key 16 beta + 4 grp + j: P's operand is the lane's
+//     own p, V's one dword of row 4 grp + j.
+// The next tile's K and V come from memory into registers while this one is used, its block
+// ids one tile earlier still. LDS rows are padded by 16 bytes: K's 16-byte reads of 16 keys
+// and V's dwords of 4 rows x 16 dims then fall on distinct banks. The halves' states merge
+// through LDS at the end.
+// Bound by the MFMAs where the rows fill the GPU, by the tiles' latency below that. us per call,
+// before (16 tokens per workgroup, scores and P.V on the VALU, no load in flight under the
+// arithmetic) and now, fp32: 8 x 300 tokens behind up to 1,500, 32 / 8 heads, hd 128: 3,154 ->
+// 547; 3 x 100-300 behind up to 700, hd 128: 371 -> 83; 1,000 tokens, hd 64: 234 -> 62; 20
+// behind 2,000: 54 -> 17; 2 x 100-300, hd 256: 144 -> 68; bf16 at hd 16, 4 x 100-400: 93 -> 16.
+// Error against 64 bits on 3 chunks of 60-300 tokens, hd 64: 3.5e-7 -> 3.2e-7.
 // ---------------------------------------------------------------------------------
 
-template <int HD> struct RowsShape {
-  static constexpr int TK = HD >= 256 ? 32 : 64;  // keys per tile
-  static constexpr int KS = kWave / TK;            // lane groups splitting head_dim
-  static constexpr int DPL = HD >= kWave ? HD / kWave : 1;  // head dims per lane (P.V)
-  static constexpr int TOK = 16;                   // query tokens per workgroup
-  static constexpr int TPW = 4;                    // query tokens per wave
+template <int HD> struct F32Shape {
+  static constexpr int TK = HD <= 64 ? 64 : (HD == 128 ? 32 : 16);  // keys per tile
+  static constexpr int NB = TK / 16;    // 16-key blocks per tile
+  static constexpr int LDW = HD + 4;    // floats per staged row
+  static constexpr int DTL = HD / 16;   // 16-dim tiles of O^T
+  static constexpr int BM = 64;         // query rows per workgroup
 };
 
-template <int DT, int HD, int GPW>
-__global__ void __launch_bounds__(256)
-paged_prefill_rows_kernel(const PrefillArgs a) {
-  using SH = RowsShape<HD>;
-  constexpr int TK = SH::TK, KS = SH::KS, DPL = SH::DPL, TOK = SH::TOK, TPW = SH::TPW;
-  constexpr int P = TPW * GPW;
+template <int DT, int HD>
+__global__ void __launch_bounds__(512)
+paged_prefill_f32_kernel(const PrefillArgs a) {
+  using SH = F32Shape<HD>;
+  constexpr int TK = SH::TK, NB = SH::NB, LDW = SH::LDW, DTL = SH::DTL, BM = SH::BM;
   constexpr int VEC = vec16<DT>();
-  constexpr int CPR = HD / VEC;  // 16-byte chunks per K/V row
+  constexpr int CPR = HD / VEC;                       // 16-byte chunks per K/V row
+  constexpr int NL = (TK * CPR + 255) / 256;          // chunks per thread of a half, K and V each
   using S = typename Elt<DT>::S;
-  __shared__ float ks[TK][HD + 1];  // padded: lane j reads row j conflict-free
-  __shared__ float vs[TK][HD];
-  __shared__ int live[TK];
-  __shared__ __attribute__((aligned(16))) float qs[4][P][HD];
-  __shared__ __attribute__((aligned(16))) float es[4][P][TK];
+  __shared__ __align__(16) float kv[2][2][TK][LDW];   // [half][K, V]
+  __shared__ __align__(16) int live[2][TK];
+  __shared__ float xml[4][2][kWave];                  // the merge's (m, l)
 
-  const int lane = threadIdx.x & (kWave - 1);
-  const int wave = threadIdx.x / kWave;
-  const int tiles = (int)gridDim.x / a.n_chunks;  // query tiles per chunk (static bound)
-  const int c = blockIdx.x / tiles;
-  const int tt = blockIdx.x - c * tiles;
-  const int nsub = (a.groups + GPW - 1) / GPW;
-  const int kvh = blockIdx.y / nsub;
-  const int h0 = kvh * a.groups + (blockIdx.y - kvh * nsub) * GPW;
-  const int hend = (kvh + 1) * a.groups;  // heads of this KV head end here
+  const int tid = threadIdx.x, htid = tid & 255;
+  const int half = __builtin_amdgcn_readfirstlane(tid >> 8);
+  const int lane = tid & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(htid / kWave);
+  const int col = lane & 15, grp = lane >> 4;
+  const PrefillItem it = pick_item(a, (int)blockIdx.x);
+  const int c = it.c, q0 = it.q0, n = it.n, kvh = it.kvh;
+  const int qlen = it.q1 - q0, G = a.groups, nrows = qlen * G;
+  const int rho0 = (a.row_blocks - 1 - it.rbi) * BM;
+  if (qlen <= 0 || rho0 >= nrows) return;  // uniform per workgroup
+  const int base_pos = n - qlen;
 
-  const int q0 = a.cu_q[c], ql = a.cu_q[c + 1] - q0;
-  if (tt * TOK >= ql) return;  // workgroup-uniform
-  int n = a.ctx[c];
-  const int cap = a.max_blocks * a.bs;
-  n = n < 0 ? 0 : (n > cap ? cap : n);
-  const int last_tok = min(ql, (tt + 1) * TOK) - 1;  // last valid token of the tile
-  // Keys the tile's queries may see: 0 .. kmax - 1.
-  const int kmax = a.causal ? max(0, min(n, n - ql + last_tok + 1)) : n;
-
-  // This wave's pairs: pair p = (token i = p / GPW, head h0 + p % GPW).
-  const int tok0 = tt * TOK + TPW * wave;
-  for (int e = lane; e < P * HD; e += kWave) {
-    const int p = e / HD, d = e - p * HD;
-    const int i = tok0 + p / GPW, h = h0 + p % GPW;
-    float x = 0.f;
-    int64_t row = -1;
-    if (i < ql) row = a.rows ? token_row(a, q0 + i) : a.q_rows ? a.q_rows[q0 + i] : q0 + i;
-    if (row >= 0 && h < hend)  // a negative q_rows entry: no query there
-      x = Elt<DT>::to_f32(reinterpret_cast<const S*>(a.q)[row * a.q_st +
-                                                        (int64_t)h * a.q_sh + d]);
-    qs[wave][p][d] = x * a.scale_log2;
-  }
-  int qpos[TPW];  // position of each token of the wave (keys <= qpos are visible)
+  // This lane's query row: its token, head, place in q and out, and its visible keys.
+  const int rho = rho0 + 16 * wave + col;
+  const int tok = min(rho, nrows - 1) / G, head = kvh * G + min(rho, nrows - 1) % G;
+  int64_t qrow = q0 + tok;
+  if (a.rows) qrow = token_row(a, qrow);
+  else if (a.q_rows) qrow = a.q_rows[q0 + tok];
+  const bool row_ok = rho < nrows && qrow >= 0;  // no query: nothing read or written
+  const int64_t orow = a.rows ? qrow : q0 + tok;
+  float qf[HD / 16][4];
+  {
+    const S* qp = reinterpret_cast<const S*>(a.q) + (row_ok ? qrow : 0) * a.q_st +
+                  (int64_t)head * a.q_sh + 4 * grp;
 #pragma unroll
-  for (int i = 0; i < TPW; ++i) qpos[i] = a.causal ? n - ql + tok0 + i : n - 1;
-
-  float m[P], l[P], acc[P][DPL];
+    for (int i = 0; i < HD / 16; ++i) {
+      S x[4];
+      if constexpr (DT == PKV_F32) *reinterpret_cast<float4*>(x) = *reinterpret_cast<const float4*>(qp + 16 * i);
+      else *reinterpret_cast<uint2*>(x) = *reinterpret_cast<const uint2*>(qp + 16 * i);
 #pragma unroll
-  for (int p = 0; p < P; ++p) {
-    m[p] = -INFINITY;
-    l[p] = 0.f;
-#pragma unroll
-    for (int k = 0; k < DPL; ++k) acc[p][k] = 0.f;
-  }
-  const int j = lane % TK;    // this lane's key in the score phase
-  const int part = lane / TK; // which share of head_dim it sums (KS > 1)
-  const int64_t head_off = (int64_t)kvh * a.kv_sh;
-
-  for (int kt = 0; kt < kmax; kt += TK) {
-    __syncthreads();  // the previous tile's readers are done
-    for (int e = threadIdx.x; e < TK * CPR; e += blockDim.x) {
-      const int r = e / CPR, ch = e - r * CPR;
-      const int pos = kt + r;
-      int64_t slot = -1;
-      if (pos < kmax) {
-        const int blk = a.bs_shift >= 0 ? pos >> a.bs_shift : pos / a.bs;
-        const int64_t sl = (int64_t)a.tables[(int64_t)c * a.table_stride + blk] * a.bs +
-                           (pos - blk * a.bs);
-        slot = (sl >= 0 && sl < a.num_slots) ? sl : -1;
-      }
-      float kf[VEC], vf[VEC];
-      if (slot >= 0) {
-        const int64_t off = slot * a.kv_ss + head_off + ch * VEC;
-        unpack16<DT>(*reinterpret_cast<const uint4*>(reinterpret_cast<const S*>(a.k) + off), kf);
-        unpack16<DT>(*reinterpret_cast<const uint4*>(reinterpret_cast<const S*>(a.v) + off), vf);
-      } else {
-#pragma unroll
-        for (int i = 0; i < VEC; ++i) kf[i] = vf[i] = 0.f;
-      }
-#pragma unroll
-      for (int i = 0; i < VEC; ++i) {
-        ks[r][ch * VEC + i] = kf[i];
-        vs[r][ch * VEC + i] = vf[i];
-      }
-      if (ch == 0) live[r] = slot >= 0;
+      for (int j = 0; j < 4; ++j) qf[i][j] = row_ok ? Elt<DT>::to_f32(x[j]) * a.scale_log2 : 0.f;
     }
+  }
+  const int last_row = min(nrows - 1, rho0 + BM - 1);
+  const int kend = a.causal ? min(n, base_pos + last_row / G + 1) : n;  // keys any row sees
+  const int limit = a.causal ? min(n - 1, base_pos + tok) : n - 1;      // last key of this row
+  const int ntiles = kend > 0 ? (kend + TK - 1) / TK : 0;
+  const int ns = (ntiles + 1) / 2;
+  const int tbeg = half ? ns : 0, nt = half ? ntiles - ns : ns;
+
+  // Staging: chunk e = htid + 256 i of a tile is 16 bytes of row e / CPR.
+  const int32_t* trow = a.tables + (int64_t)c * a.table_stride;
+  auto blk_of = [&](int p) { return a.bs_shift >= 0 ? p >> a.bs_shift : p / a.bs; };
+  int bid[NL];
+  auto load_ids = [&](int m) {  // block ids of local tile m's rows
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+      const int p = (tbeg + m) * TK + (htid + 256 * i) / CPR;
+      bid[i] = m < nt && p < kend ? trow[blk_of(p)] : -1;
+    }
+  };
+  uint4 kr[NL], vr[NL];
+  bool ok[NL];
+  auto load_kv = [&](int m) {
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+      const int e = htid + 256 * i;
+      const int p = (tbeg + m) * TK + e / CPR;
+      const int64_t sl = (int64_t)bid[i] * a.bs + (p - blk_of(p) * a.bs);
+      ok[i] = (TK * CPR % 256 == 0 || e < TK * CPR) && m < nt && p < kend && bid[i] >= 0 &&
+              sl < a.num_slots;
+      kr[i] = vr[i] = make_uint4(0, 0, 0, 0);
+      if (ok[i]) {
+        const int64_t off = sl * a.kv_ss + (int64_t)kvh * a.kv_sh + (e % CPR) * VEC;
+        kr[i] = *reinterpret_cast<const uint4*>(reinterpret_cast<const S*>(a.k) + off);
+        vr[i] = *reinterpret_cast<const uint4*>(reinterpret_cast<const S*>(a.v) + off);
+      }
+    }
+  };
+  auto store_kv = [&]() {
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+      const int e = htid + 256 * i;
+      if (TK * CPR % 256 != 0 && e >= TK * CPR) break;
+      const int r = e / CPR, ch = e % CPR;
+      float f[VEC];
+      unpack16<DT>(kr[i], f);
+      store_vec<PKV_F32, VEC>(&kv[half][0][r][ch * VEC], f);
+      unpack16<DT>(vr[i], f);
+      store_vec<PKV_F32, VEC>(&kv[half][1][r][ch * VEC], f);
+      if (ch == 0) live[half][r] = ok[i];
+    }
+  };
+
+  float m_run = -INFINITY, l_run = 0.f;  // of row col (l: this lane's keys)
+  f32x4 ov[DTL];                         // O^T: dims 16 d + 4 grp + r of row col
+#pragma unroll
+  for (int d = 0; d < DTL; ++d) ov[d] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  load_ids(0);
+  load_kv(0);
+  load_ids(1);
+  for (int m = 0; m < ns; ++m) {  // both halves pass every barrier
+    __syncthreads();              // the previous tile's readers are done
+    if (m < nt) store_kv();
     __syncthreads();
-
-    // Scores of key kt + j for every pair.
-    float sc[P];
+    if (m >= nt) continue;
+    load_kv(m + 1);
+    load_ids(m + 2);
+    f32x4 sc[NB];
 #pragma unroll
-    for (int p = 0; p < P; ++p) sc[p] = 0.f;
-    constexpr int DS = HD / KS;  // head dims per lane share
-#pragma unroll 2
-    for (int d = part * DS; d < (part + 1) * DS; d += 4) {
-      const float k0 = ks[j][d], k1 = ks[j][d + 1], k2 = ks[j][d + 2], k3 = ks[j][d + 3];
+    for (int b = 0; b < NB; ++b) sc[b] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int p = 0; p < P; ++p) {
-        const float4 qv = *reinterpret_cast<const float4*>(&qs[wave][p][d]);
-        sc[p] = __builtin_fmaf(k0, qv.x, __builtin_fmaf(k1, qv.y,
-                 __builtin_fmaf(k2, qv.z, __builtin_fmaf(k3, qv.w, sc[p]))));
+    for (int i = 0; i < HD / 16; ++i) {
+      f32x4 kf[NB];
+#pragma unroll
+      for (int b = 0; b < NB; ++b)
+        kf[b] = *reinterpret_cast<const f32x4*>(&kv[half][0][16 * b + col][16 * i + 4 * grp]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+          sc[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[b][j], qf[i][j], sc[b], 0, 0, 0);
+    }
+    float mx = -INFINITY;
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      const int4 lv = *reinterpret_cast<const int4*>(&live[half][16 * b + 4 * grp]);
+      const int on[4] = {lv.x, lv.y, lv.z, lv.w};
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int kpos = (tbeg + m) * TK + 16 * b + 4 * grp + r;
+        sc[b][r] = on[r] && kpos <= limit ? sc[b][r] : -INFINITY;
+        mx = fmaxf(mx, sc[b][r]);
       }
     }
-    const int kpos = kt + j;
-    const bool key_ok = kpos < kmax && live[j];
+    const float mn = fmaxf(m_run, rows_max(mx));
+    const float mref = mn == -INFINITY ? 0.f : mn;  // nothing visible yet: stay at 0
+    const float alpha = __builtin_amdgcn_exp2f(m_run - mref);
+    m_run = mn;
+    l_run *= alpha;
 #pragma unroll
-    for (int p = 0; p < P; ++p) {
-      if constexpr (KS > 1) sc[p] += __shfl_xor(sc[p], TK);
-      const bool vis = key_ok && kpos <= qpos[p / GPW];
-      const float s = vis ? sc[p] : -INFINITY;
-      const float mx = across_max<1>(s);  // the same for every lane
-      const float mn = fmaxf(m[p], mx);
-      const float mref = mn == -INFINITY ? 0.f : mn;  // nothing visible yet: stay at 0
-      const float alpha = __builtin_amdgcn_exp2f(m[p] - mref);
-      const float pr = __builtin_amdgcn_exp2f(s - mref);
-      m[p] = mn;
-      l[p] = l[p] * alpha + (part == 0 ? pr : 0.f);
+    for (int d = 0; d < DTL; ++d) ov[d] *= alpha;
 #pragma unroll
-      for (int k = 0; k < DPL; ++k) acc[p][k] *= alpha;
-      if (part == 0) es[wave][p][j] = pr;
-    }
-    __syncthreads();
-
-    // P.V: lane d accumulates head dims d + 64 k.
-#pragma unroll 2
-    for (int jj = 0; jj < TK; jj += 4) {
-      float vv[4][DPL];
+    for (int b = 0; b < NB; ++b)
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
-#pragma unroll
-        for (int k = 0; k < DPL; ++k)
-          vv[r][k] = (lane + kWave * k < HD) ? vs[jj + r][lane + kWave * k] : 0.f;
-#pragma unroll
-      for (int p = 0; p < P; ++p) {
-        const float4 w = *reinterpret_cast<const float4*>(&es[wave][p][jj]);
-#pragma unroll
-        for (int k = 0; k < DPL; ++k)
-          acc[p][k] = __builtin_fmaf(w.x, vv[0][k], __builtin_fmaf(w.y, vv[1][k],
-                      __builtin_fmaf(w.z, vv[2][k], __builtin_fmaf(w.w, vv[3][k], acc[p][k]))));
+      for (int r = 0; r < 4; ++r) {
+        sc[b][r] = __builtin_amdgcn_exp2f(sc[b][r] - mref);
+        l_run += sc[b][r];
       }
-    }
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int d = 0; d < DTL; ++d)
+          ov[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[half][1][16 * b + 4 * grp + j][16 * d + col],
+                                                       sc[b][j], ov[d], 0, 0, 0);
   }
+  float l_tot = rows_sum(l_run);
 
+  // Merge the halves: half 1 leaves (m, l, O^T) per lane, half 0's same lane takes them.
+  static_assert(4 * DTL * 4 * kWave <= 2 * 2 * TK * LDW, "the exchange fits the staged tiles");
+  float* x = &kv[0][0][0][0] + wave * DTL * 4 * kWave + lane;
+  __syncthreads();
+  if (half) {
+    xml[wave][0][lane] = m_run;
+    xml[wave][1][lane] = l_tot;
 #pragma unroll
-  for (int p = 0; p < P; ++p) {
-    const float lt = across_sum_exact<1>(l[p]);
-    const int i = tok0 + p / GPW, h = h0 + p % GPW;
-    if (i >= ql || h >= hend || (a.q_rows && a.q_rows[q0 + i] < 0)) continue;
-    const float inv = lt > 0.f ? 1.f / lt : 0.f;  // nothing visible: 0
-    const int64_t t = q0 + i;
-    const int64_t orow = a.rows ? token_row(a, t) : t;
-    if (orow < 0) continue;
+    for (int d = 0; d < DTL; ++d)
 #pragma unroll
-    for (int k = 0; k < DPL; ++k) {
-      const int d = lane + kWave * k;
-      if (d >= HD) break;
-      const int64_t e = orow * a.out_st + (int64_t)h * a.out_sh + d;
-      const float o = acc[p][k] * inv;
-      if (a.out_f32) reinterpret_cast<float*>(a.out)[e] = o;
-      else reinterpret_cast<S*>(a.out)[e] = Elt<DT>::from_f32(o);
-    }
-    if (a.lse && lane == 0) a.lse[t * a.nh + h] = lt > 0.f ? m[p] + __log2f(lt) : -INFINITY;
+      for (int r = 0; r < 4; ++r) x[(4 * d + r) * kWave] = ov[d][r];
   }
+  __syncthreads();
+  if (half || !row_ok) return;
+  const float mb = xml[wave][0][lane];
+  const float mn = fmaxf(m_run, mb);
+  const float mref = mn == -INFINITY ? 0.f : mn;  // both empty: weights 0
+  const float sa = __builtin_amdgcn_exp2f(m_run - mref), sb = __builtin_amdgcn_exp2f(mb - mref);
+  l_tot = l_tot * sa + xml[wave][1][lane] * sb;
+  const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;  // nothing visible: 0
+  const int64_t e0 = orow * a.out_st + (int64_t)head * a.out_sh + 4 * grp;
+#pragma unroll
+  for (int d = 0; d < DTL; ++d) {
+    float o[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) o[r] = (ov[d][r] * sa + x[(4 * d + r) * kWave] * sb) * inv;
+    if (a.out_f32) store_vec<PKV_F32, 4>((float*)a.out + e0 + 16 * d, o);
+    else store_vec<DT, 4>((S*)a.out + e0 + 16 * d, o);
+  }
+  if (a.lse && grp == 0)
+    a.lse[(int64_t)(q0 + tok) * a.nh + head] = l_tot > 0.f ? mn + __log2f(l_tot) : -INFINITY;
 }
 
 // ---------------------------------------------------------------------------------
@@ -259,32 +298,21 @@ hipError_t launch_v16(const PrefillArgs& a, int hd, hipStream_t st) {
   return hipGetLastError();
 }
 
-// The VALU kernel: grid (chunks x query tiles, KV heads x head sub-groups).
-template <int DT, int HD, int GPW>
-hipError_t launch_rows_gpw(const PrefillArgs& a, int max_query_len, hipStream_t st) {
-  constexpr int TOK = RowsShape<HD>::TOK;
-  const int64_t tiles = (max_query_len + TOK - 1) / TOK;
-  const int64_t x = tiles * a.n_chunks;
-  const int64_t y = (int64_t)a.nkv * ((a.groups + GPW - 1) / GPW);
-  if (x > 0x7FFFFFFF || y > 65535) return hipErrorInvalidValue;
-  hipLaunchKernelGGL((paged_prefill_rows_kernel<DT, HD, GPW>), dim3((unsigned)x, (unsigned)y),
-                     dim3(256), 0, st, a);
+// The fp32 kernel: one workgroup per item (chunk, 64-row block, KV head).
+template <int DT, int HD> hipError_t launch_f32_hd(PrefillArgs a, int64_t rows, hipStream_t st) {
+  a.row_blocks = (int)((rows + F32Shape<HD>::BM - 1) / F32Shape<HD>::BM);
+  const int64_t items = (int64_t)a.row_blocks * a.nkv * a.n_chunks;
+  if (items > 0x7FFFFFFF) return hipErrorInvalidValue;
+  hipLaunchKernelGGL((paged_prefill_f32_kernel<DT, HD>), dim3((unsigned)items), dim3(512), 0, st, a);
   return hipGetLastError();
 }
-template <int DT, int HD>
-hipError_t launch_rows_hd(const PrefillArgs& a, int max_query_len, hipStream_t st) {
-  if (a.groups == 1) return launch_rows_gpw<DT, HD, 1>(a, max_query_len, st);
-  if (a.groups == 2) return launch_rows_gpw<DT, HD, 2>(a, max_query_len, st);
-  return launch_rows_gpw<DT, HD, 4>(a, max_query_len, st);
-}
-template <int DT>
-hipError_t launch_rows(const PrefillArgs& a, int hd, int max_query_len, hipStream_t st) {
+hipError_t launch_f32(const PrefillArgs& a, int hd, int64_t rows, hipStream_t st) {
   switch (hd) {
-    case 16: return launch_rows_hd<DT, 16>(a, max_query_len, st);
-    case 32: return launch_rows_hd<DT, 32>(a, max_query_len, st);
-    case 64: return launch_rows_hd<DT, 64>(a, max_query_len, st);
-    case 128: return launch_rows_hd<DT, 128>(a, max_query_len, st);
-    default: return launch_rows_hd<DT, 256>(a, max_query_len, st);
+    case 16: return launch_f32_hd<PKV_F32, 16>(a, rows, st);
+    case 32: return launch_f32_hd<PKV_F32, 32>(a, rows, st);
+    case 64: return launch_f32_hd<PKV_F32, 64>(a, rows, st);
+    case 128: return launch_f32_hd<PKV_F32, 128>(a, rows, st);
+    default: return launch_f32_hd<PKV_F32, 256>(a, rows, st);
   }
 }
 
@@ -365,15 +393,13 @@ int prefill_args(PrefillArgs* out_args, int64_t* rows_out, void* out, int out_dt
 
 namespace {
 
-// Launches for checked arguments: the matrix cores take 16-bit K/V at head_dim 32..256
-// (a bf16 call with a.v16 set converts the chunks' V first), the VALU kernel the rest.
-int run_prefill(const PrefillArgs& a, int64_t rows, int kv_dtype, int head_dim,
-                int max_query_len, hipStream_t st) {
-  if (kv_dtype == PKV_F32) return (int)launch_rows<PKV_F32>(a, head_dim, max_query_len, st);
-  if (head_dim == 16) {
-    return (int)(kv_dtype == PKV_BF16 ? launch_rows<PKV_BF16>(a, head_dim, max_query_len, st)
-                                      : launch_rows<PKV_F16>(a, head_dim, max_query_len, st));
-  }
+// Launches for checked arguments: the 16-bit matrix-core kernel takes 16-bit K/V at head_dim
+// 32..256 (a bf16 call with a.v16 set converts the chunks' V first), the fp32 kernel the rest.
+int run_prefill(const PrefillArgs& a, int64_t rows, int kv_dtype, int head_dim, hipStream_t st) {
+  if (kv_dtype == PKV_F32) return (int)launch_f32(a, head_dim, rows, st);
+  if (head_dim == 16)
+    return (int)(kv_dtype == PKV_BF16 ? launch_f32_hd<PKV_BF16, 16>(a, rows, st)
+                                      : launch_f32_hd<PKV_F16, 16>(a, rows, st));
   if (kv_dtype == PKV_F16)
     return (int)(a.rows ? launch_prefill<PKV_F16, true>(a, head_dim, rows, st)
                         : launch_prefill<PKV_F16, false>(a, head_dim, rows, st));
@@ -446,7 +472,7 @@ int pkv_paged_prefill_ex(void* out, int out_dtype, int64_t out_stride_tok, int64
                                max_query_len, num_heads, num_kv_heads, head_dim, block_size,
                                scale, causal, q_rows, lse);
   if (bad) return bad == 1 ? 0 : bad;
-  return run_prefill(a, rows, kv_dtype, head_dim, max_query_len, (hipStream_t)stream);
+  return run_prefill(a, rows, kv_dtype, head_dim, (hipStream_t)stream);
 }
 
 int64_t pkv_prefill_workspace_bytes(int kv_dtype, int32_t head_dim, int32_t num_kv_heads,
@@ -514,7 +540,7 @@ int pkv_paged_prefill_rows(void* out, int out_dtype, int64_t out_stride_tok, int
       a.v16 = static_cast<const char*>(workspace) + l.k_bytes;
     }
   }
-  return run_prefill(a, qrows, kv_dtype, head_dim, max_query_len, (hipStream_t)stream);
+  return run_prefill(a, qrows, kv_dtype, head_dim, (hipStream_t)stream);
 }
 
 }  // extern "C"

@@ -1112,9 +1112,8 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs& a, const Prefill
 // exit is workgroup-uniform except half 1's after the merge; a caller that runs several
 // items on one workgroup puts a barrier between them (the merge reuses the rings).
 // V16: V from the fp16 copy (bf16 caches; the launch guarantees every chunk's region).
-template <int DT, int HD, bool POW2, bool V16, bool ROWS>
-__device__ __forceinline__ void prefill_item(const PrefillArgs& a, const int item,
-                                             PrefillLds<HD>& lds) {
+// The coordinates of item `item`.
+__device__ __forceinline__ PrefillItem pick_item(const PrefillArgs& a, const int item) {
   const int lane = threadIdx.x & (kWave - 1);
   // Work items (chunk, row block, KV head), heaviest first: chunks by context length
   // (longest first), then row blocks from the last (it sees the most keys), KV heads
@@ -1147,7 +1146,13 @@ __device__ __forceinline__ void prefill_item(const PrefillArgs& a, const int ite
     it.q1 = a.cu_q[it.c + 1];
     it.n = min(max(a.ctx[it.c], 0), cap);
   }
-  prefill_body<DT, HD, POW2, V16, ROWS>(a, it, lds);
+  return it;
+}
+
+template <int DT, int HD, bool POW2, bool V16, bool ROWS>
+__device__ __forceinline__ void prefill_item(const PrefillArgs& a, const int item,
+                                             PrefillLds<HD>& lds) {
+  prefill_body<DT, HD, POW2, V16, ROWS>(a, pick_item(a, item), lds);
 }
 
 // Head_dim 32 and 64 leave room for two workgroups on a CU (72 KB of LDS each at 64): the

@@ -642,8 +642,7 @@ def paged_prefill_attention(
     ``max_query_len`` bounds every chunk (it sizes the grid: one graph per bucket).
     16-bit caches at head_dim 32-256 run on the matrix cores (the reference's
     FlashAttention shapes); fp32 caches and head_dim 16 (the reference's per-chunk SDPA
-    path, layers.py:254-265) on a VALU kernel that stages each K/V tile in LDS once per
-    16 query tokens. For bf16 caches the call first writes each chunk's V as fp16 (per
+    path, layers.py:254-265) on their fp32 instructions (fp32 products and sums). For bf16 caches the call first writes each chunk's V as fp16 (per
     256-token tile scaled by a power of two that keeps it inside fp16's range) into a
     workspace, so that P enters the second product once, in fp16, instead of as a bf16
     hi + lo pair; ``workspace`` (a CUDA byte tensor of at least

@@ -1,0 +1,57 @@
+"""Chunked prefill in fp32 arithmetic (fp32 caches, and 16-bit ones at head_dim 16) against
+attention in float64, at the edges of its tiles: 64 query rows, 16 / 32 / 64 keys, two halves."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from engine import workloads
+from engine.kernels import paged_attention as pa
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda:0")
+# |V| < 6 times fp32 scores of a few ulps (|s| < 16) and fp32 sums
+TOL = 6 * 16 * 2.0**-22
+
+
+def _exact(step, lens):
+    q, k, v = step_q(step), step.k_cache.cpu().double(), step.v_cache.cpu().double()
+    g, bs = q.shape[1] // k.shape[1], step.block_size
+    out, at = torch.zeros(q.shape, dtype=torch.float64), 0
+    for c, (m, n) in enumerate(zip(lens, step.context_lens.tolist(), strict=True)):
+        p = torch.arange(n)
+        slots = step.block_tables[c].cpu().long()[p // bs] * bs + p % bs
+        kb, vb = (x[slots].repeat_interleave(g, 1).transpose(0, 1) for x in (k, v))
+        s = (q[at : at + m].transpose(0, 1) @ kb.transpose(1, 2)) * q.shape[-1] ** -0.5
+        s = s.masked_fill(p[None, None] > (n - m + torch.arange(m))[None, :, None], float("-inf"))
+        out[at : at + m] = (torch.softmax(s, -1) @ vb).transpose(0, 1)
+        at += m
+    return out
+
+
+def step_q(step):
+    return step.info["q"].cpu().double()
+
+
+@pytest.mark.parametrize(("hd", "dtype"), [(16, torch.float32), (32, torch.float32), (64, torch.float32),
+                                           (128, torch.float32), (256, torch.float32),
+                                           (16, torch.bfloat16), (16, torch.float16)])  # fmt: skip
+@pytest.mark.parametrize(("nh", "nkv", "bs"), [(4, 4, 16), (6, 2, 5), (8, 2, 16), (7, 1, 64)])
+def test_tile_edges(nh, nkv, bs, hd, dtype):
+    lens = [1, 15, 16, 17, 64, 65, 9, 33]
+    cached = [0, 0, 16, 111, 1, 0, 500, 31]
+    step = workloads.custom([a + b for a, b in zip(lens, cached, strict=True)], nh, nkv, hd, bs,
+                            dtype, DEV, seed=hd)  # fmt: skip
+    q = torch.randn(sum(lens), nh, hd, device=DEV).to(dtype)
+    step.info["q"] = q
+    cu = torch.tensor([0, *torch.tensor(lens).cumsum(0).tolist()], dtype=torch.int32, device=DEV)
+    print("[case] prefill f32", nh, nkv, hd, bs, dtype, flush=True)
+    out = torch.full(q.shape, float("nan"), device=DEV)
+    args = (step.k_cache, step.v_cache, step.block_tables, step.context_lens, bs, cu, max(lens))
+    pa.paged_prefill_attention(q, *args, out=out)
+    rounded = pa.paged_prefill_attention(q, *args)
+    torch.cuda.synchronize()
+    err = (out.cpu().double() - _exact(step, lens)).abs().max().item()
+    assert err <= TOL, err
+    assert torch.equal(rounded, out.to(dtype))
