@@ -391,6 +391,20 @@ int pkv_rms_norm(void* out, int out_dtype, int64_t out_stride_row, const void* x
                  int64_t rows, int64_t cols, void* stream);
 
 /*
+ * pkv_rms_norm from the rows' means of squares (fp32 [rows], PyTorch's mean): the row scale is
+ * 1 / sqrt(mean + eps), the sum rounded to fp32, the rest in fp64 rounded to fp32 -- the bits of
+ * PyTorch's ROCm rsqrt on every non-negative value.
+ */
+int pkv_rms_norm_mean(void* out, int out_dtype, int64_t out_stride_row, const void* x, int x_dtype,
+                      int64_t x_stride_row, const float* mean, float eps, const void* weight,
+                      int w_dtype, int64_t rows, int64_t cols, void* stream);
+
+/* out[r, c] = x[r, c]^2 in fp32, out contiguous [rows, cols]: x.float().pow(2) in one pass, for
+ * that mean. */
+int pkv_square(float* out, const void* x, int dtype, int64_t x_stride_row, int64_t rows,
+               int64_t cols, void* stream);
+
+/*
  * RoPE in place (reference fused.py:61-80, :114-121): x [n_tokens, heads, head_dim]
  * (unit stride in head_dim) becomes x * cos + rotate_half(x) * sin, rotate_half(x) =
  * cat(-x[half:], x[:half]); cos / sin are fp32 [n_tokens, head_dim] with row stride

@@ -7,9 +7,10 @@
 // bitwise identical to them: every product and sum is one fp32 operation rounded to the
 // tensor dtype at the points PyTorch rounds, exp and division are the device library's
 // and IEEE (as in PyTorch's ROCm SiLU), and multiply-add contraction is off for the whole
-// file (PyTorch's separate kernels round between the multiply and the add). RMSNorm
-// takes its per-row scale rsqrt(mean(x^2) + eps) from the caller: the device library's
-// rsqrtf and PyTorch's ROCm rsqrt can differ in the last fp32 bit.
+// file (PyTorch's separate kernels round between the multiply and the add). RMSNorm leaves
+// the mean of its squares to PyTorch (a sum in another order has other bits); its rsqrt is
+// 1 / sqrt(x) in fp64 rounded to fp32, which is what PyTorch's ROCm rsqrt gives on every
+// non-negative fp32 value (the device library's rsqrtf differs on 11% of them).
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -55,8 +56,12 @@ template <int DT> __device__ __forceinline__ float through(float f) {
 
 // 16 bytes of DT: VN<DT> elements (8 of a 16-bit type, 4 floats).
 template <int DT> constexpr int VN = DT == PKV_F32 ? 4 : 8;
-template <int DT> __device__ __forceinline__ void load16(const typename F<DT>::S* p, float* f) {
-  const uint4 r = *reinterpret_cast<const uint4*>(p);
+// NT: non-temporal, for data too large to be found in the caches again.
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+template <int DT, bool NT = false>
+__device__ __forceinline__ void load16(const typename F<DT>::S* p, float* f) {
+  const u32x4* q = reinterpret_cast<const u32x4*>(p);
+  const u32x4 r = NT ? __builtin_nontemporal_load(q) : *q;
   const uint32_t w[4] = {r.x, r.y, r.z, r.w};
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
@@ -68,16 +73,51 @@ template <int DT> __device__ __forceinline__ void load16(const typename F<DT>::S
     }
   }
 }
-template <int DT> __device__ __forceinline__ void store16(typename F<DT>::S* p, const float* f) {
-  uint32_t w[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    if constexpr (DT == PKV_F32)
-      w[i] = __float_as_uint(f[i]);
-    else
-      w[i] = (uint32_t)F<DT>::down(f[2 * i]) | ((uint32_t)F<DT>::down(f[2 * i + 1]) << 16);
+// Two values rounded to a 16-bit DT, packed. bf16 through v_cvt_pk_bf16_f32, which rounds every
+// value as down() does but keeps the bits of a NaN.
+template <int DT> __device__ __forceinline__ uint32_t pack2(float a, float b) {
+  if constexpr (DT == PKV_BF16) {
+    typedef __bf16 v2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, v2{(__bf16)a, (__bf16)b});
+  } else {
+    return (uint32_t)F<DT>::down(a) | ((uint32_t)F<DT>::down(b) << 16);
   }
-  *reinterpret_cast<uint4*>(p) = make_uint4(w[0], w[1], w[2], w[3]);
+}
+// f[0 .. N) after a cast to DT and back (through()), in place; the bits of NaNs aside, which
+// the store of whatever is computed from them sets.
+template <int DT, int N> __device__ __forceinline__ void round_all(float* f) {
+  if constexpr (DT != PKV_F32) {
+#pragma unroll
+    for (int i = 0; i < N; i += 2) {
+      const uint32_t w = pack2<DT>(f[i], f[i + 1]);
+      f[i] = F<DT>::up((uint16_t)(w & 0xFFFFu));
+      f[i + 1] = F<DT>::up((uint16_t)(w >> 16));
+    }
+  }
+}
+template <int DT, bool NT = false>
+__device__ __forceinline__ void store16(typename F<DT>::S* p, const float* f) {
+  uint32_t w[4];
+  if constexpr (DT == PKV_F32) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) w[i] = __float_as_uint(f[i]);
+  } else {
+    bool nan = false;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      w[i] = pack2<DT>(f[2 * i], f[2 * i + 1]);
+      nan = nan || __builtin_isunordered(f[2 * i], f[2 * i + 1]);
+    }
+    if (DT == PKV_BF16 && nan) {  // PyTorch's one NaN
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        w[i] = (uint32_t)F<DT>::down(f[2 * i]) | ((uint32_t)F<DT>::down(f[2 * i + 1]) << 16);
+    }
+  }
+  u32x4* q = reinterpret_cast<u32x4*>(p);
+  const u32x4 v = {w[0], w[1], w[2], w[3]};
+  if constexpr (NT) __builtin_nontemporal_store(v, q);
+  else *q = v;
 }
 // n fp32 values (n a multiple of 4) from a 16-byte aligned address.
 template <int N> __device__ __forceinline__ void load_f32(const float* p, float* f) {
@@ -88,16 +128,25 @@ template <int N> __device__ __forceinline__ void load_f32(const float* p, float*
   }
 }
 
+// A row's scale: the caller's inv_rms, or rsqrt(mean + eps) from its mean of squares.
+struct RowScale {
+  const float* v;
+  float eps;
+  bool mean;
+  __device__ __forceinline__ float at(int64_t r) const {
+    return mean ? (float)(1.0 / sqrt((double)(v[r] + eps))) : v[r];
+  }
+};
+
 // out[r, c] = DO( f32(w[c]) * f32(DX( f32(x[r, c]) * inv[r] )) ): PyTorch's
 // w * (x.float() * inv).to(x.dtype), inv = torch.rsqrt(mean(x.float()^2) + eps) per row.
 template <int DX, int DW, int DO>
 __global__ void __launch_bounds__(256)
 rms_norm_tail_kernel(typename F<DO>::S* __restrict__ out, int64_t so,
-                     const typename F<DX>::S* __restrict__ x, int64_t sx,
-                     const float* __restrict__ inv_rms, const typename F<DW>::S* __restrict__ w,
-                     int64_t rows, int cols) {
+                     const typename F<DX>::S* __restrict__ x, int64_t sx, const RowScale scale,
+                     const typename F<DW>::S* __restrict__ w, int64_t rows, int cols) {
   for (int64_t r = blockIdx.y; r < rows; r += gridDim.y) {
-    const float inv = inv_rms[r];
+    const float inv = scale.at(r);
     for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < cols; c += gridDim.x * blockDim.x) {
       const float normed = through<DX>(F<DX>::up(x[r * sx + c]) * inv);
       out[r * so + c] = F<DO>::down(F<DW>::up(w[c]) * normed);
@@ -150,61 +199,132 @@ silu_mul_kernel(typename F<DT>::S* __restrict__ out, const typename F<DT>::S* __
 // The same three operations, 16 bytes per access (x, weight and output of one dtype for
 // the RMSNorm tail; the launchers take these when pointers, strides and widths allow).
 // Each element goes through exactly the scalar kernels' operations.
+// One workgroup per row at a time; its first wave computes the row's scale (fp64: once per
+// workgroup, not per thread) while the row's first loads are in flight.
 template <int DT>
 __global__ void __launch_bounds__(256)
 rms_norm_tail_vec_kernel(typename F<DT>::S* __restrict__ out, int64_t so,
                          const typename F<DT>::S* __restrict__ x, int64_t sx,
-                         const float* __restrict__ inv_rms,
-                         const typename F<DT>::S* __restrict__ w, int64_t rows, int cvec) {
+                         const RowScale scale, const typename F<DT>::S* __restrict__ w,
+                         int64_t rows, int cvec) {
   constexpr int V = VN<DT>;
-  for (int64_t r = blockIdx.y; r < rows; r += gridDim.y) {
-    const float inv = inv_rms[r];
-    for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < cvec; c += gridDim.x * blockDim.x) {
-      float xf[V], wf[V], o[V];
+  __shared__ float inv_s;
+  for (int64_t r = blockIdx.x; r < rows; r += gridDim.x) {
+    int c = threadIdx.x;
+    float xf[V], wf[V], o[V];
+    if (c < cvec) {
       load16<DT>(x + r * sx + (int64_t)c * V, xf);
       load16<DT>(w + (int64_t)c * V, wf);
+    }
+    if (threadIdx.x < 64) {
+      const float inv = scale.at(r);
+      if (threadIdx.x == 0) inv_s = inv;
+    }
+    __syncthreads();
+    const float inv = inv_s;
+    __syncthreads();  // the next row's scale may be written
+    while (c < cvec) {
 #pragma unroll
-      for (int j = 0; j < V; ++j) o[j] = wf[j] * through<DT>(xf[j] * inv);
+      for (int j = 0; j < V; ++j) o[j] = xf[j] * inv;
+      round_all<DT, V>(o);
+#pragma unroll
+      for (int j = 0; j < V; ++j) o[j] = wf[j] * o[j];
       store16<DT>(out + r * so + (int64_t)c * V, o);
+      c += blockDim.x;
+      if (c < cvec) {
+        load16<DT>(x + r * sx + (int64_t)c * V, xf);
+        load16<DT>(w + (int64_t)c * V, wf);
+      }
     }
   }
 }
 
+// sq[r, c] = f32(x[r, c])^2, sq contiguous: what PyTorch's x.float().pow(2) holds, in one pass
+// (2,168 x 4,096 bf16: 8.9 us against 10.0 + 10.7 for the two).
 template <int DT>
+__global__ void __launch_bounds__(256)
+square_kernel(float* __restrict__ sq, const typename F<DT>::S* __restrict__ x, int64_t sx,
+              int64_t rows, int cols) {
+  for (int64_t r = blockIdx.y; r < rows; r += gridDim.y)
+    for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < cols; c += gridDim.x * blockDim.x) {
+      const float v = F<DT>::up(x[r * sx + c]);
+      sq[r * cols + c] = v * v;
+    }
+}
+// Four elements per access, so the fp32 stores of a wave are one contiguous piece.
+template <int DT>
+__global__ void __launch_bounds__(256)
+square_vec_kernel(float* __restrict__ sq, const typename F<DT>::S* __restrict__ x, int64_t sx,
+                  int64_t rows, int cvec) {
+  for (int64_t r = blockIdx.y; r < rows; r += gridDim.y)
+    for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < cvec; c += gridDim.x * blockDim.x) {
+      typename F<DT>::S v[4];
+      const typename F<DT>::S* p = x + r * sx + (int64_t)c * 4;
+      if constexpr (DT == PKV_F32) *reinterpret_cast<float4*>(v) = *reinterpret_cast<const float4*>(p);
+      else *reinterpret_cast<uint2*>(v) = *reinterpret_cast<const uint2*>(p);
+      float f[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) f[j] = F<DT>::up(v[j]) * F<DT>::up(v[j]);
+      reinterpret_cast<float4*>(sq + r * cvec * 4)[c] = make_float4(f[0], f[1], f[2], f[3]);
+    }
+}
+
+// A thread turns the same 2 x 16 bytes of HPT heads of one token, whose cos and sin it loads
+// and rounds once; a workgroup holds per_wg tokens of `items` threads each (or one token,
+// looped over, where a token has more items than threads). Index arithmetic is 32-bit but for
+// the row addresses (it was three 64-bit divisions per 32 bytes). Bound by memory: 2,168 tokens,
+// hd 128, bf16, 32 heads 14.6 -> 10.2 us (36 MB there and back), 8 heads 4.9 -> 4.5.
+template <int DT, int HPT>
 __global__ void __launch_bounds__(256)
 rope_vec_kernel(typename F<DT>::S* __restrict__ x, int64_t sn, int64_t sh,
                 const float* __restrict__ cs, const float* __restrict__ sn_, int64_t sc,
-                int64_t n, int heads, int half) {
+                int64_t n, int heads, int half, int items, int per_wg) {
   constexpr int V = VN<DT>;
   const int hv = half / V;
-  const int64_t total = n * heads * hv;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    const int d = (int)(i % hv) * V;
-    const int64_t nh = i / hv;
-    const int h = (int)(nh % heads);
-    const int64_t t = nh / heads;
-    typename F<DT>::S* p = x + t * sn + h * sh;
-    float x1[V], x2[V], c1[V], c2[V], s1[V], s2[V], o1[V], o2[V];
-    load16<DT>(p + d, x1);
-    load16<DT>(p + d + half, x2);
-    load_f32<V>(cs + t * sc + d, c1);
-    load_f32<V>(cs + t * sc + d + half, c2);
-    load_f32<V>(sn_ + t * sc + d, s1);
-    load_f32<V>(sn_ + t * sc + d + half, s2);
+  const int sub = (int)threadIdx.x / items;  // 0 where a token fills the workgroup
+  if (sub >= per_wg) return;
+  for (int64_t t = (int64_t)blockIdx.x * per_wg + sub; t < n; t += (int64_t)gridDim.x * per_wg) {
+    for (int i = (int)threadIdx.x - sub * items; i < items; i += 256) {
+      const int hg = i / hv, d = (i - hg * hv) * V, h0 = hg * HPT;
+      typename F<DT>::S* p = x + t * sn + h0 * sh + d;
+      float x1[HPT][V], x2[HPT][V], c1[V], c2[V], s1[V], s2[V];
 #pragma unroll
-    for (int j = 0; j < V; ++j) {
-      const float cc1 = through<DT>(c1[j]), cc2 = through<DT>(c2[j]);
-      const float ss1 = through<DT>(s1[j]), ss2 = through<DT>(s2[j]);
-      o1[j] = through<DT>(x1[j] * cc1) + through<DT>(-x2[j] * ss1);
-      o2[j] = through<DT>(x2[j] * cc2) + through<DT>(x1[j] * ss2);
+      for (int k = 0; k < HPT; ++k)
+        if (h0 + k < heads) {
+          load16<DT>(p + k * sh, x1[k]);
+          load16<DT>(p + k * sh + half, x2[k]);
+        }
+      load_f32<V>(cs + t * sc + d, c1);
+      load_f32<V>(cs + t * sc + d + half, c2);
+      load_f32<V>(sn_ + t * sc + d, s1);
+      load_f32<V>(sn_ + t * sc + d + half, s2);
+      round_all<DT, V>(c1);
+      round_all<DT, V>(c2);
+      round_all<DT, V>(s1);
+      round_all<DT, V>(s2);
+#pragma unroll
+      for (int k = 0; k < HPT; ++k)
+        if (h0 + k < heads) {
+          float a1[V], b1[V], a2[V], b2[V];
+#pragma unroll
+          for (int j = 0; j < V; ++j) {
+            a1[j] = x1[k][j] * c1[j], b1[j] = -x2[k][j] * s1[j];
+            a2[j] = x2[k][j] * c2[j], b2[j] = x1[k][j] * s2[j];
+          }
+          round_all<DT, V>(a1);
+          round_all<DT, V>(b1);
+          round_all<DT, V>(a2);
+          round_all<DT, V>(b2);
+#pragma unroll
+          for (int j = 0; j < V; ++j) a1[j] += b1[j], a2[j] += b2[j];
+          store16<DT>(p + k * sh, a1);
+          store16<DT>(p + k * sh + half, a2);
+        }
     }
-    store16<DT>(p + d, o1);
-    store16<DT>(p + d + half, o2);
   }
 }
 
-template <int DT>
+template <int DT, bool NT>
 __global__ void __launch_bounds__(256)
 silu_mul_vec_kernel(typename F<DT>::S* __restrict__ out, const typename F<DT>::S* __restrict__ g,
                     const typename F<DT>::S* __restrict__ u, int64_t nvec) {
@@ -212,11 +332,14 @@ silu_mul_vec_kernel(typename F<DT>::S* __restrict__ out, const typename F<DT>::S
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nvec;
        i += (int64_t)gridDim.x * blockDim.x) {
     float gf[V], uf[V], o[V];
-    load16<DT>(g + i * V, gf);
-    load16<DT>(u + i * V, uf);
+    load16<DT, NT>(g + i * V, gf);
+    load16<DT, NT>(u + i * V, uf);
 #pragma unroll
-    for (int j = 0; j < V; ++j) o[j] = through<DT>(gf[j] / (1.0f + expf(-gf[j]))) * uf[j];
-    store16<DT>(out + i * V, o);
+    for (int j = 0; j < V; ++j) o[j] = gf[j] / (1.0f + expf(-gf[j]));
+    round_all<DT, V>(o);
+#pragma unroll
+    for (int j = 0; j < V; ++j) o[j] *= uf[j];
+    store16<DT, NT>(out + i * V, o);
   }
 }
 
@@ -234,7 +357,7 @@ unsigned blocks_for(int64_t n) {
 }
 
 template <int DX, int DW>
-hipError_t launch_rms(void* out, int64_t so, const void* x, int64_t sx, const float* inv,
+hipError_t launch_rms(void* out, int64_t so, const void* x, int64_t sx, const RowScale& inv,
                       const void* w, int64_t rows, int cols, hipStream_t st) {
   constexpr int DO = DX == DW ? DX : PKV_F32;
   const unsigned gy = (unsigned)(rows < 65535 ? rows : 65535);
@@ -243,8 +366,8 @@ hipError_t launch_rms(void* out, int64_t so, const void* x, int64_t sx, const fl
     if (cols % V == 0 && sx % V == 0 && so % V == 0 && aligned16(out) && aligned16(x) &&
         aligned16(w)) {
       const int cvec = cols / V;
-      hipLaunchKernelGGL((rms_norm_tail_vec_kernel<DX>), dim3((unsigned)((cvec + 255) / 256), gy),
-                         dim3(256), 0, st, (typename F<DX>::S*)out, so,
+      const unsigned gr = (unsigned)(rows < 0x7FFFFFFF ? rows : 0x7FFFFFFF);
+      hipLaunchKernelGGL((rms_norm_tail_vec_kernel<DX>), dim3(gr), dim3(256), 0, st, (typename F<DX>::S*)out, so,
                          (const typename F<DX>::S*)x, sx, inv, (const typename F<DX>::S*)w, rows,
                          cvec);
       return hipGetLastError();
@@ -258,7 +381,7 @@ hipError_t launch_rms(void* out, int64_t so, const void* x, int64_t sx, const fl
 }
 
 template <int DX>
-hipError_t rms_by_w(int dw, void* out, int64_t so, const void* x, int64_t sx, const float* inv,
+hipError_t rms_by_w(int dw, void* out, int64_t so, const void* x, int64_t sx, const RowScale& inv,
                     const void* w, int64_t rows, int cols, hipStream_t st) {
   switch (dw) {
     case PKV_F32: return launch_rms<DX, PKV_F32>(out, so, x, sx, inv, w, rows, cols, st);
@@ -267,18 +390,68 @@ hipError_t rms_by_w(int dw, void* out, int64_t so, const void* x, int64_t sx, co
   }
 }
 
-}  // namespace
+// Streaming accesses where the output alone is larger than the L2s (8 x 4 MB), so that the next
+// kernel would not find it there either: 2,168 x 14,336 bf16 31.1 us against 34.7-36.9 (186 MB,
+// 6.0 TB/s); streaming loads alone 35.2-36.7.
+constexpr int64_t kStreamBytes = 32 << 20;
+template <int DT>
+hipError_t launch_silu(void* out, const void* g, const void* u, int64_t nvec, hipStream_t st) {
+  using S = typename F<DT>::S;
+  const unsigned nb = blocks_for(nvec);
+  if (nvec * 16 >= kStreamBytes)
+    hipLaunchKernelGGL((silu_mul_vec_kernel<DT, true>), dim3(nb), dim3(256), 0, st, (S*)out,
+                       (const S*)g, (const S*)u, nvec);
+  else
+    hipLaunchKernelGGL((silu_mul_vec_kernel<DT, false>), dim3(nb), dim3(256), 0, st, (S*)out,
+                       (const S*)g, (const S*)u, nvec);
+  return hipGetLastError();
+}
 
-extern "C" {
+// Heads per thread of the vector RoPE: 4 once that leaves at least 128 Ki threads (two waves per
+// SIMD of 256 CUs), else 1 (more threads in flight).
+template <int DT, int HPT>
+hipError_t launch_rope_hpt(void* x, int64_t sn, int64_t sh, const float* cs, const float* sn_,
+                           int64_t sc, int64_t n, int heads, int half, hipStream_t st) {
+  const int64_t items = (int64_t)((heads + HPT - 1) / HPT) * (half / VN<DT>);
+  if (items > 0x7FFFFFFF) return hipErrorInvalidValue;
+  const int per = items < 256 ? (int)(256 / items) : 1;
+  const int64_t wgs = (n + per - 1) / per;
+  hipLaunchKernelGGL((rope_vec_kernel<DT, HPT>), dim3((unsigned)(wgs < 0x7FFFFFFF ? wgs : 0x7FFFFFFF)),
+                     dim3(256), 0, st, (typename F<DT>::S*)x, sn, sh, cs, sn_, sc, n, heads, half,
+                     (int)items, per);
+  return hipGetLastError();
+}
+template <int DT>
+hipError_t launch_rope(void* x, int64_t sn, int64_t sh, const float* cs, const float* sn_,
+                       int64_t sc, int64_t n, int heads, int half, hipStream_t st) {
+  if (n * heads * (half / VN<DT>) >= (int64_t)4 << 17)
+    return launch_rope_hpt<DT, 4>(x, sn, sh, cs, sn_, sc, n, heads, half, st);
+  return launch_rope_hpt<DT, 1>(x, sn, sh, cs, sn_, sc, n, heads, half, st);
+}
 
-int pkv_rms_norm(void* out, int out_dtype, int64_t out_stride_row, const void* x, int x_dtype,
-                 int64_t x_stride_row, const float* inv_rms, const void* weight, int w_dtype,
-                 int64_t rows, int64_t cols, void* stream) {
+template <int DT>
+hipError_t launch_square(float* sq, const void* x, int64_t sx, int64_t rows, int cols,
+                         hipStream_t st) {
+  const unsigned gy = (unsigned)(rows < 65535 ? rows : 65535);
+  if (cols % 4 == 0 && sx % 4 == 0 && aligned16(sq) && aligned16(x)) {
+    const int cvec = cols / 4;
+    hipLaunchKernelGGL((square_vec_kernel<DT>), dim3((unsigned)((cvec + 255) / 256), gy), dim3(256),
+                       0, st, sq, (const typename F<DT>::S*)x, sx, rows, cvec);
+  } else {
+    hipLaunchKernelGGL((square_kernel<DT>), dim3((unsigned)((cols + 255) / 256), gy), dim3(256), 0,
+                       st, sq, (const typename F<DT>::S*)x, sx, rows, cols);
+  }
+  return hipGetLastError();
+}
+
+int rms_norm(void* out, int out_dtype, int64_t out_stride_row, const void* x, int x_dtype,
+             int64_t x_stride_row, const RowScale& inv_rms, const void* weight, int w_dtype,
+             int64_t rows, int64_t cols, void* stream) {
   if (!valid(x_dtype) || !valid(w_dtype) || out_dtype != promoted(x_dtype, w_dtype))
     return PKV_E_DTYPE;
   if (rows < 0 || cols < 0 || cols > (1 << 30)) return PKV_E_SHAPE;
   if (rows == 0 || cols == 0) return 0;
-  if (!out || !x || !inv_rms || !weight) return PKV_E_NULL;
+  if (!out || !x || !inv_rms.v || !weight) return PKV_E_NULL;
   hipStream_t st = (hipStream_t)stream;
   const int c = (int)cols;
   switch (x_dtype) {
@@ -294,6 +467,38 @@ int pkv_rms_norm(void* out, int out_dtype, int64_t out_stride_row, const void* x
   }
 }
 
+}  // namespace
+
+extern "C" {
+
+int pkv_rms_norm(void* out, int out_dtype, int64_t out_stride_row, const void* x, int x_dtype,
+                 int64_t x_stride_row, const float* inv_rms, const void* weight, int w_dtype,
+                 int64_t rows, int64_t cols, void* stream) {
+  return rms_norm(out, out_dtype, out_stride_row, x, x_dtype, x_stride_row,
+                  RowScale{inv_rms, 0.f, false}, weight, w_dtype, rows, cols, stream);
+}
+
+int pkv_rms_norm_mean(void* out, int out_dtype, int64_t out_stride_row, const void* x, int x_dtype,
+                      int64_t x_stride_row, const float* mean, float eps, const void* weight,
+                      int w_dtype, int64_t rows, int64_t cols, void* stream) {
+  return rms_norm(out, out_dtype, out_stride_row, x, x_dtype, x_stride_row,
+                  RowScale{mean, eps, true}, weight, w_dtype, rows, cols, stream);
+}
+
+int pkv_square(float* out, const void* x, int dtype, int64_t x_stride_row, int64_t rows,
+               int64_t cols, void* stream) {
+  if (!valid(dtype)) return PKV_E_DTYPE;
+  if (rows < 0 || cols < 0 || cols > (1 << 30)) return PKV_E_SHAPE;
+  if (rows == 0 || cols == 0) return 0;
+  if (!out || !x) return PKV_E_NULL;
+  hipStream_t st = (hipStream_t)stream;
+  switch (dtype) {
+    case PKV_F32: return (int)launch_square<PKV_F32>(out, x, x_stride_row, rows, (int)cols, st);
+    case PKV_F16: return (int)launch_square<PKV_F16>(out, x, x_stride_row, rows, (int)cols, st);
+    default: return (int)launch_square<PKV_BF16>(out, x, x_stride_row, rows, (int)cols, st);
+  }
+}
+
 int pkv_rope(void* x, int dtype, int64_t stride_tok, int64_t stride_head, const float* cos,
              const float* sin, int64_t cs_stride_tok, int64_t n_tokens, int32_t heads,
              int32_t head_dim, void* stream) {
@@ -306,21 +511,17 @@ int pkv_rope(void* x, int dtype, int64_t stride_tok, int64_t stride_head, const 
   const int v = dtype == PKV_F32 ? 4 : 8;  // elements per 16-byte access
   if (half % v == 0 && stride_tok % v == 0 && stride_head % v == 0 && cs_stride_tok % 4 == 0 &&
       aligned16(x) && aligned16(cos) && aligned16(sin)) {
-    const unsigned nbv = blocks_for(n_tokens * heads * (half / v));
     switch (dtype) {
       case PKV_F32:
-        hipLaunchKernelGGL(rope_vec_kernel<PKV_F32>, dim3(nbv), dim3(256), 0, st, (float*)x,
-                           stride_tok, stride_head, cos, sin, cs_stride_tok, n_tokens, heads, half);
-        break;
+        return (int)launch_rope<PKV_F32>(x, stride_tok, stride_head, cos, sin, cs_stride_tok,
+                                         n_tokens, heads, half, st);
       case PKV_F16:
-        hipLaunchKernelGGL(rope_vec_kernel<PKV_F16>, dim3(nbv), dim3(256), 0, st, (uint16_t*)x,
-                           stride_tok, stride_head, cos, sin, cs_stride_tok, n_tokens, heads, half);
-        break;
+        return (int)launch_rope<PKV_F16>(x, stride_tok, stride_head, cos, sin, cs_stride_tok,
+                                         n_tokens, heads, half, st);
       default:
-        hipLaunchKernelGGL(rope_vec_kernel<PKV_BF16>, dim3(nbv), dim3(256), 0, st, (uint16_t*)x,
-                           stride_tok, stride_head, cos, sin, cs_stride_tok, n_tokens, heads, half);
+        return (int)launch_rope<PKV_BF16>(x, stride_tok, stride_head, cos, sin, cs_stride_tok,
+                                          n_tokens, heads, half, st);
     }
-    return (int)hipGetLastError();
   }
   const unsigned nb = blocks_for(n_tokens * heads * half);
   switch (dtype) {
@@ -348,21 +549,11 @@ int pkv_silu_mul(void* out, const void* gate, const void* up, int dtype, int64_t
   hipStream_t st = (hipStream_t)stream;
   const int v = dtype == PKV_F32 ? 4 : 8;  // elements per 16-byte access
   if (n % v == 0 && aligned16(out) && aligned16(gate) && aligned16(up)) {
-    const unsigned nbv = blocks_for(n / v);
     switch (dtype) {
-      case PKV_F32:
-        hipLaunchKernelGGL(silu_mul_vec_kernel<PKV_F32>, dim3(nbv), dim3(256), 0, st,
-                           (float*)out, (const float*)gate, (const float*)up, n / v);
-        break;
-      case PKV_F16:
-        hipLaunchKernelGGL(silu_mul_vec_kernel<PKV_F16>, dim3(nbv), dim3(256), 0, st,
-                           (uint16_t*)out, (const uint16_t*)gate, (const uint16_t*)up, n / v);
-        break;
-      default:
-        hipLaunchKernelGGL(silu_mul_vec_kernel<PKV_BF16>, dim3(nbv), dim3(256), 0, st,
-                           (uint16_t*)out, (const uint16_t*)gate, (const uint16_t*)up, n / v);
+      case PKV_F32: return (int)launch_silu<PKV_F32>(out, gate, up, n / v, st);
+      case PKV_F16: return (int)launch_silu<PKV_F16>(out, gate, up, n / v, st);
+      default: return (int)launch_silu<PKV_BF16>(out, gate, up, n / v, st);
     }
-    return (int)hipGetLastError();
   }
   const unsigned nb = blocks_for(n);
   switch (dtype) {

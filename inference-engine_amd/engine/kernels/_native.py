@@ -72,6 +72,11 @@ SIGNATURES: dict[str, tuple] = {
         ctypes.c_int,
         [_p, ctypes.c_int, _i64, _p, ctypes.c_int, _i64, _p, _p, ctypes.c_int, _i64, _i64, _p],
     ),  # fmt: skip
+    "pkv_rms_norm_mean": (
+        ctypes.c_int,
+        [_p, ctypes.c_int, _i64, _p, ctypes.c_int, _i64, _p, _f32, _p, ctypes.c_int, _i64, _i64, _p],
+    ),  # fmt: skip
+    "pkv_square": (ctypes.c_int, [_p, _p, ctypes.c_int, _i64, _i64, _i64, _p]),
     "pkv_rope": (ctypes.c_int, [_p, ctypes.c_int, _i64, _i64, _p, _p, _i64, _i64, _i32, _i32, _p]),
     "pkv_silu_mul": (ctypes.c_int, [_p, _p, _p, ctypes.c_int, _i64, _p]),
     "pkv_paged_decode_ex": (

@@ -1,11 +1,11 @@
 """Fused element-wise kernels beside the paged path: RMSNorm tail, in-place RoPE and
-SiLU-and-multiply, one HIP launch each (csrc/fused.hip through lib/libpaged_kv.so).
+SiLU-and-multiply (csrc/fused.hip through lib/libpaged_kv.so).
 Same names, signatures and contract as the reference's ``engine/kernels/fused.py``
 (:38-131): every result is bitwise identical to the PyTorch ops it replaces, rounding
 where they round, with the device library's exp and IEEE division and no multiply-add
-contraction. RMSNorm leaves the per-row scale rsqrt(mean(x^2) + eps) to PyTorch: the
-reference leaves it the mean (a fused sum adds in another order), and on ROCm PyTorch's
-rsqrt can differ from the device library's in the last fp32 bit.
+contraction. RMSNorm leaves the mean of its squares to PyTorch, as the reference does (a
+fused sum adds in another order): one launch squares, PyTorch's mean reduces, one launch
+scales, with PyTorch's rsqrt bits.
 """
 
 from __future__ import annotations
@@ -43,13 +43,17 @@ def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
     weight = weight.contiguous()
     if weight.shape != (shape[-1],):
         raise ValueError(f"{what}: weight {tuple(weight.shape)} for rows of {shape[-1]}")
-    inv = torch.rsqrt(x2.float().pow(2).mean(-1) + eps)
+    rows, cols = x2.shape
+    code, stream, lib = _native.dtype_code(x.dtype, what), _native.stream_of(dev), _native.lib()
+    sq = torch.empty((rows, cols), dtype=torch.float32, device=dev)
+    _native.check(lib.pkv_square(sq.data_ptr(), x2.data_ptr(), code, x2.stride(0), rows, cols,
+                                 stream), what)  # fmt: skip
+    mean = sq.mean(-1)
     out = torch.empty(x2.shape, dtype=torch.promote_types(weight.dtype, x.dtype), device=dev)
-    status = _native.lib().pkv_rms_norm(
+    status = lib.pkv_rms_norm_mean(
         out.data_ptr(), _native.dtype_code(out.dtype, what), out.stride(0),
-        x2.data_ptr(), _native.dtype_code(x.dtype, what), x2.stride(0), inv.data_ptr(),
-        weight.data_ptr(), _native.dtype_code(weight.dtype, what), x2.shape[0], x2.shape[1],
-        _native.stream_of(dev))  # fmt: skip
+        x2.data_ptr(), code, x2.stride(0), mean.data_ptr(), float(eps), weight.data_ptr(),
+        _native.dtype_code(weight.dtype, what), rows, cols, stream)  # fmt: skip
     _native.check(status, what)
     return out.view(shape)
 
