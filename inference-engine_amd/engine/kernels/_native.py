@@ -194,8 +194,14 @@ def dtype_code(dtype: torch.dtype, what: str) -> int:
         raise TypeError(f"{what}: unsupported dtype {dtype}") from None
 
 
+# The current stream's handle without building a Stream object (0.1 us against 1.9 us).
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream_of(device: torch.device) -> int:
     """hipStream_t of torch's current stream on ``device`` (captured into graphs as-is)."""
+    if _raw_stream is not None and device.index is not None:
+        return _raw_stream(device.index)
     return torch.cuda.current_stream(device).cuda_stream
 
 
@@ -257,7 +263,15 @@ def check_tables(what: str, block_tables: torch.Tensor, context_lens: torch.Tens
 
 
 def require_gpu(what: str, *tensors: torch.Tensor) -> torch.device:
-    dev = tensors[0].device
+    first = tensors[0]
+    dev = first.device
+    if first.is_cuda:
+        index = first.get_device()
+        for t in tensors:
+            if not t.is_cuda or t.get_device() != index:
+                break
+        else:
+            return dev
     if dev.type != "cuda":
         raise ValueError(f"{what}: tensors must be on a GPU device, got {dev}")
     for t in tensors[1:]:

@@ -28,6 +28,7 @@ of ``_native.set_debug_checks`` excepted).
 
 from __future__ import annotations
 
+import functools
 from collections.abc import Sequence
 from dataclasses import dataclass
 
@@ -380,10 +381,11 @@ def paged_decode_attention(
     what = "paged_decode_attention"
     dev = _check_decode_args(what, q, k_cache, v_cache, block_tables, context_lens, block_size,
                              rows)  # fmt: skip
-    b = q.shape[0] if rows is None else rows.numel()
-    _, nh, hd = q.shape
-    nkv = k_cache.shape[1]
-    kv_code = _native.dtype_code(k_cache.dtype, what)
+    n_rows, nh, hd = q.shape
+    b = n_rows if rows is None else rows.numel()
+    num_slots, nkv, _ = k_cache.shape
+    dtype = q.dtype
+    kv_code = _native.dtype_code(dtype, what)
 
     if rows is None:
         q = q.contiguous()
@@ -400,7 +402,7 @@ def paged_decode_attention(
 
     max_blocks = block_tables.shape[1]
     lib = _native.lib()
-    cascade = prefix_groups is not None and q.dtype in (torch.bfloat16, torch.float16) \
+    cascade = prefix_groups is not None and dtype in (torch.bfloat16, torch.float16) \
         and hd in PREFILL_HEAD_DIMS  # fmt: skip
     if cascade:
         _check_prefix_groups(prefix_groups, b, dev, what)
@@ -408,10 +410,9 @@ def paged_decode_attention(
     # workspace), else the stream-K split over decode_workgroups() workgroups.
     wg_arg = 0 if num_workgroups is None else num_workgroups
     if num_workgroups is None:
-        num_workgroups = decode_workgroups(dev, q.dtype, hd, nh, nkv) if cascade else \
-            default_workgroups(dev, q.dtype, hd, nh, nkv, b, max_blocks, block_size)  # fmt: skip
-    query = lib.pkv_cascade_workspace_bytes if cascade else lib.pkv_decode_workspace_bytes
-    ws_bytes = query(num_workgroups, b, nh, hd) if num_workgroups else 0
+        num_workgroups = decode_workgroups(dev, dtype, hd, nh, nkv) if cascade else \
+            default_workgroups(dev, dtype, hd, nh, nkv, b, max_blocks, block_size)  # fmt: skip
+    ws_bytes = _workspace_bytes(num_workgroups, b, nh, hd, cascade) if num_workgroups else 0
     ws = None
     if ws_bytes and workspace is not None:
         if workspace.device != dev or workspace.dtype != torch.uint8 or \
@@ -421,12 +422,13 @@ def paged_decode_attention(
         ws = workspace
     elif ws_bytes:
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+    q_sb, q_sh, _ = q.stride()
+    out_sb, out_sh, _ = out.stride()
+    kv_ss, kv_sh, _ = k_cache.stride()
     common = (
-        out.data_ptr(), _native.dtype_code(out.dtype, what), out.stride(0), out.stride(1),
-        q.data_ptr(), q.stride(0), q.stride(1),
-        k_cache.data_ptr(), v_cache.data_ptr(), kv_code,
-        k_cache.stride(0), k_cache.stride(1), k_cache.shape[0],
-        block_tables.data_ptr(), block_tables.stride(0), max_blocks,
+        out.data_ptr(), kv_code if out.dtype is dtype else _native.PKV_F32, out_sb, out_sh,
+        q.data_ptr(), q_sb, q_sh, k_cache.data_ptr(), v_cache.data_ptr(), kv_code,
+        kv_ss, kv_sh, num_slots, block_tables.data_ptr(), block_tables.stride(0), max_blocks,
         context_lens.data_ptr(), b, nh, nkv, hd, block_size,
         hd**-0.5, wg_arg, ws.data_ptr() if ws is not None else None, ws_bytes,
     )  # fmt: skip
@@ -444,13 +446,21 @@ def paged_decode_attention(
             pg.prefix_row.data_ptr(), pg.pieces, pg.members, pwg, _native.stream_of(dev),
         )  # fmt: skip
     elif rows is not None:
-        status = lib.pkv_paged_decode_rows(*common, rows.data_ptr(), q.shape[0],
+        status = lib.pkv_paged_decode_rows(*common, rows.data_ptr(), n_rows,
                                            _native.stream_of(dev))  # fmt: skip
     else:
-        status = lib.pkv_paged_decode_ex(*common, None, None, None, None, None, 0, 0,
-                                         _native.stream_of(dev))  # fmt: skip
-    _native.check(status, what)
+        status = lib.pkv_paged_decode(*common, _native.stream_of(dev))
+    if status:
+        _native.check(status, what)
     return out
+
+
+@functools.lru_cache(maxsize=1024)
+def _workspace_bytes(num_workgroups: int, batch: int, num_heads: int, head_dim: int,
+                     cascade: bool) -> int:  # fmt: skip
+    lib = _native.lib()
+    query = lib.pkv_cascade_workspace_bytes if cascade else lib.pkv_decode_workspace_bytes
+    return query(num_workgroups, batch, num_heads, head_dim)
 
 
 def paged_decode_attention_noalloc(
@@ -536,27 +546,31 @@ def _check_decode_args(what, q, k_cache, v_cache, block_tables, context_lens,
                        block_size, rows=None) -> torch.device:  # fmt: skip
     """The decode entry points' argument checks (before any launch); returns the device."""
     dev = _native.require_gpu(what, q, k_cache, v_cache, block_tables, context_lens)
-    if q.dim() != 3 or k_cache.dim() != 3 or v_cache.dim() != 3:
+    qs, ks = q.shape, k_cache.shape
+    if len(qs) != 3 or len(ks) != 3 or v_cache.dim() != 3:
         raise ValueError(f"{what}: q, k_cache, v_cache must be 3-D")
-    b, nh, hd = q.shape
+    b, nh, hd = qs
     if rows is not None:
         b = rows.numel()
-    nkv = k_cache.shape[1]
-    if v_cache.shape != k_cache.shape or k_cache.shape[2] != hd:
-        raise ValueError(f"{what}: cache shapes {tuple(k_cache.shape)}, "
-                         f"{tuple(v_cache.shape)} do not match q {tuple(q.shape)}")  # fmt: skip
+    nkv = ks[1]
+    if v_cache.shape != ks or ks[2] != hd:
+        raise ValueError(f"{what}: cache shapes {tuple(ks)}, "
+                         f"{tuple(v_cache.shape)} do not match q {tuple(qs)}")  # fmt: skip
     if nh % nkv:
         raise ValueError(f"{what}: {nh} query heads not a multiple of {nkv} KV heads")
     if hd not in SUPPORTED_HEAD_DIMS:
         raise ValueError(f"{what}: head_dim {hd} not in {SUPPORTED_HEAD_DIMS}")
-    if q.dtype != k_cache.dtype or v_cache.dtype != k_cache.dtype:
-        raise TypeError(f"{what}: q {q.dtype} and caches {k_cache.dtype}/{v_cache.dtype} "
+    dtype = k_cache.dtype
+    if q.dtype != dtype or v_cache.dtype != dtype:
+        raise TypeError(f"{what}: q {q.dtype} and caches {dtype}/{v_cache.dtype} "
                         "must share one dtype")  # fmt: skip
-    if k_cache.stride() != v_cache.stride() or k_cache.stride(2) != 1:
+    kst = k_cache.stride()
+    if kst != v_cache.stride() or kst[2] != 1:
         raise ValueError(f"{what}: k_cache and v_cache need equal strides, unit in head_dim")
     if block_tables.dtype != torch.int32 or context_lens.dtype != torch.int32:
         raise TypeError(f"{what}: block_tables and context_lens must be int32")
-    if block_tables.dim() != 2 or block_tables.shape[0] != b or block_tables.stride(1) != 1:
+    ts = block_tables.shape
+    if len(ts) != 2 or ts[0] != b or block_tables.stride(1) != 1:
         raise ValueError(f"{what}: block_tables must be [B, max_blocks] with unit column stride")
     if context_lens.shape != (b,) or not context_lens.is_contiguous():
         raise ValueError(f"{what}: context_lens must be a contiguous [B] tensor")
@@ -694,28 +708,36 @@ def paged_prefill_attention(
                       cu_seqlens_q, t, max_query_len)  # fmt: skip
     context_lens = context_lens.contiguous()
     cu_seqlens_q = cu_seqlens_q.contiguous()
-    kv_code = _native.dtype_code(k_cache.dtype, what)
+    dtype = k_cache.dtype
+    kv_code = _native.dtype_code(dtype, what)
+    max_blocks = block_tables.shape[1]
+    ws_ptr, ws_bytes = None, 0
     if workspace is None:
-        need = prefill_workspace_bytes(k_cache.dtype, hd, nkv, n_chunks, block_tables.shape[1],
-                                       block_size)  # fmt: skip
+        need = prefill_workspace_bytes(dtype, hd, nkv, n_chunks, max_blocks, block_size)
         if 0 < need <= PREFILL_WORKSPACE_MAX_BYTES:
             workspace = torch.empty(need, dtype=torch.uint8, device=dev)
     elif not workspace.is_contiguous() or workspace.device != dev:
         raise ValueError(f"{what}: workspace must be a contiguous tensor on {dev}")
-    ws_ptr = workspace.data_ptr() if workspace is not None else None
-    ws_bytes = workspace.numel() * workspace.element_size() if workspace is not None else 0
-    status = _native.lib().pkv_paged_prefill_rows(
-        out.data_ptr(), _native.dtype_code(out.dtype, what), out.stride(0), out.stride(1),
-        q.data_ptr(), q.stride(0), q.stride(1),
-        k_cache.data_ptr(), v_cache.data_ptr(), kv_code,
-        k_cache.stride(0), k_cache.stride(1), k_cache.shape[0],
-        block_tables.data_ptr(), block_tables.stride(0), block_tables.shape[1],
+    if workspace is not None:
+        ws_ptr, ws_bytes = workspace.data_ptr(), workspace.numel() * workspace.element_size()
+    q_st, q_sh, _ = q.stride()
+    out_st, out_sh, _ = out.stride()
+    kv_ss, kv_sh, _ = k_cache.stride()
+    args = (
+        out.data_ptr(), _native.dtype_code(out.dtype, what), out_st, out_sh,
+        q.data_ptr(), q_st, q_sh, k_cache.data_ptr(), v_cache.data_ptr(), kv_code,
+        kv_ss, kv_sh, k_cache.shape[0], block_tables.data_ptr(), block_tables.stride(0), max_blocks,
         context_lens.data_ptr(), cu_seqlens_q.data_ptr(), n_chunks, int(max_query_len),
         nh, nkv, hd, block_size, hd**-0.5, ws_ptr, ws_bytes,
-        None if rows is None else rows.data_ptr(), 0 if rows is None else t,
-        0 if rows is None else q.shape[0], _native.stream_of(dev),
     )  # fmt: skip
-    _native.check(status, what)
+    lib = _native.lib()
+    if rows is None:
+        status = lib.pkv_paged_prefill_ws(*args, _native.stream_of(dev))
+    else:
+        status = lib.pkv_paged_prefill_rows(*args, rows.data_ptr(), t, q.shape[0],
+                                            _native.stream_of(dev))  # fmt: skip
+    if status:
+        _native.check(status, what)
     return out
 
 
@@ -727,6 +749,12 @@ def prefill_workspace_bytes(dtype: torch.dtype, head_dim: int, num_kv_heads: int
                             n_chunks: int, max_blocks: int, block_size: int) -> int:
     """Workspace bytes with which a prefill call of these static shapes writes the fp16
     copy of every chunk's V (0: the shapes take none; pkv_prefill_workspace_bytes)."""
+    return _prefill_workspace_bytes(dtype, head_dim, num_kv_heads, n_chunks, max_blocks, block_size)
+
+
+@functools.lru_cache(maxsize=1024)
+def _prefill_workspace_bytes(dtype: torch.dtype, head_dim: int, num_kv_heads: int,
+                             n_chunks: int, max_blocks: int, block_size: int) -> int:  # fmt: skip
     n = _native.lib().pkv_prefill_workspace_bytes(
         _native.DTYPE_CODE.get(dtype, -1), head_dim, num_kv_heads, n_chunks, max_blocks,
         block_size)  # fmt: skip
