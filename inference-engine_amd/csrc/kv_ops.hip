@@ -11,7 +11,11 @@ using namespace pkv;
 // KV append.
 // ---------------------------------------------------------------------------------
 
-template <int DIN, int DOUT, int VEC>
+// One thread per VEC elements of a new row. The row's slot and its data are one memory trip:
+// the data does not wait for the slot (a row without a slot is read and dropped). I: index type
+// of the grid's flat index, 32-bit where it fits (a 64-bit division per thread cost ~100
+// instructions).
+template <int DIN, int DOUT, int VEC, typename I>
 __global__ void __launch_bounds__(256)
 kv_append_kernel(typename Elt<DOUT>::S* __restrict__ k_pool,
                  typename Elt<DOUT>::S* __restrict__ v_pool, int64_t ps_slot,
@@ -22,40 +26,43 @@ kv_append_kernel(typename Elt<DOUT>::S* __restrict__ k_pool,
                  int64_t n_tokens, int nkv, int hd) {
   using SI = typename Elt<DIN>::S;
   using SO = typename Elt<DOUT>::S;
-  const int chunks = hd / VEC;
-  const int64_t per_tok = (int64_t)2 * nkv * chunks;
-  const int64_t total = n_tokens * per_tok;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t tok = i / per_tok;
-    int r = (int)(i - tok * per_tok);
-    const int c = r % chunks;
+  const unsigned chunks = (unsigned)(hd / VEC), heads = (unsigned)nkv;
+  const I per_tok = (I)2 * heads * chunks;
+  const I total = (I)n_tokens * per_tok;
+  for (I i = (I)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (I)gridDim.x * blockDim.x) {
+    const I tok = i / per_tok;
+    unsigned r = (unsigned)(i - tok * per_tok);
+    const unsigned c = r % chunks;
     r /= chunks;
-    const int head = r % nkv;
-    const bool is_v = r >= nkv;
+    const bool is_v = r >= heads;
+    const unsigned head = is_v ? r - heads : r;
     const int64_t slot = slots[tok];
-    if (slot < 0 || slot >= num_slots) continue;
-    const SI* src = is_v ? v_new + tok * vs_tok + head * vs_head
-                         : k_new + tok * ks_tok + head * ks_head;
-    SO* dst = (is_v ? v_pool : k_pool) + slot * ps_slot + head * ps_head;
+    const SI* src = is_v ? v_new + (int64_t)tok * vs_tok + head * vs_head
+                         : k_new + (int64_t)tok * ks_tok + head * ks_head;
     src += c * VEC;
-    dst += c * VEC;
-    if constexpr (DIN == DOUT && VEC * sizeof(SI) % 16 == 0) {
+    constexpr int NQ = VEC * (int)sizeof(SI) / 16;  // 16-byte pieces
+    if constexpr (NQ >= 1) {
+      uint4 q[NQ];
 #pragma unroll
-      for (int j = 0; j < (int)(VEC * sizeof(SI) / 16); ++j)
-        reinterpret_cast<uint4*>(dst)[j] = reinterpret_cast<const uint4*>(src)[j];
-    } else if constexpr (DIN == DOUT) {
+      for (int j = 0; j < NQ; ++j) q[j] = reinterpret_cast<const uint4*>(src)[j];
+      if (slot < 0 || slot >= num_slots) continue;
+      SO* dst = (is_v ? v_pool : k_pool) + slot * ps_slot + head * ps_head + c * VEC;
+      if constexpr (DIN == DOUT) {
 #pragma unroll
-      for (int j = 0; j < VEC; ++j) dst[j] = src[j];
+        for (int j = 0; j < NQ; ++j) reinterpret_cast<uint4*>(dst)[j] = q[j];
+      } else {
+        float f[VEC];
+#pragma unroll
+        for (int j = 0; j < NQ; ++j) unpack16<DIN>(q[j], f + j * (VEC / NQ));
+        store_vec<DOUT, VEC>(dst, f);
+      }
     } else {
-      SI in[VEC];
-      SO o[VEC];
-#pragma unroll
-      for (int j = 0; j < VEC; ++j) in[j] = src[j];
-#pragma unroll
-      for (int j = 0; j < VEC; ++j) o[j] = Elt<DOUT>::from_f32(Elt<DIN>::to_f32(in[j]));
-#pragma unroll
-      for (int j = 0; j < VEC; ++j) dst[j] = o[j];
+      static_assert(VEC == 1, "whole 16-byte pieces or single elements");
+      const SI x = *src;
+      if (slot < 0 || slot >= num_slots) continue;
+      SO* dst = (is_v ? v_pool : k_pool) + slot * ps_slot + head * ps_head + c;
+      if constexpr (DIN == DOUT) *dst = x;
+      else *dst = Elt<DOUT>::from_f32(Elt<DIN>::to_f32(x));
     }
   }
 }
@@ -146,11 +153,19 @@ hipError_t launch_append(void* kp, void* vp, int64_t ps_slot, int64_t ps_head,
   const int64_t total = n_tokens * 2 * nkv * (hd / VEC);
   int64_t blocks = (total + 255) / 256;
   if (blocks > 65535 * 8) blocks = 65535 * 8;
-  hipLaunchKernelGGL((kv_append_kernel<DIN, DOUT, VEC>), dim3((unsigned)blocks), dim3(256), 0,
-                     st, (typename Elt<DOUT>::S*)kp, (typename Elt<DOUT>::S*)vp, ps_slot,
-                     ps_head, num_slots, (const typename Elt<DIN>::S*)kn, ks_tok, ks_head,
-                     (const typename Elt<DIN>::S*)vn, vs_tok, vs_head, slots, n_tokens, nkv,
-                     hd);
+  // the grid-stride index may run up to one grid past the end
+  if (total + blocks * 256 <= 0xFFFFFFFFll)
+    hipLaunchKernelGGL((kv_append_kernel<DIN, DOUT, VEC, uint32_t>), dim3((unsigned)blocks), dim3(256), 0,
+                       st, (typename Elt<DOUT>::S*)kp, (typename Elt<DOUT>::S*)vp, ps_slot,
+                       ps_head, num_slots, (const typename Elt<DIN>::S*)kn, ks_tok, ks_head,
+                       (const typename Elt<DIN>::S*)vn, vs_tok, vs_head, slots, n_tokens, nkv,
+                       hd);
+  else
+    hipLaunchKernelGGL((kv_append_kernel<DIN, DOUT, VEC, int64_t>), dim3((unsigned)blocks), dim3(256), 0,
+                       st, (typename Elt<DOUT>::S*)kp, (typename Elt<DOUT>::S*)vp, ps_slot,
+                       ps_head, num_slots, (const typename Elt<DIN>::S*)kn, ks_tok, ks_head,
+                       (const typename Elt<DIN>::S*)vn, vs_tok, vs_head, slots, n_tokens, nkv,
+                       hd);
   return hipGetLastError();
 }
 
