@@ -154,8 +154,9 @@ int pkv_paged_decode(void* out, int out_dtype, int64_t out_stride_b, int64_t out
  * that forbid allocation). No counterpart in the reference: its Triton decode needs no
  * scratch. Same arguments, kernels and results as pkv_paged_decode at the same
  * num_workgroups; the split-K workspace is a static device array of
- * PKV_NOALLOC_SCRATCH_BYTES per GPU, held until the process ends. Calls whose workspace
- * (pkv_decode_workspace_bytes) exceeds it return PKV_E_SCRATCH before any launch. The
+ * PKV_NOALLOC_SCRATCH_BYTES per GPU, held until the process ends. The default split
+ * (num_workgroups 0) takes at most as many ranges as it holds; a given count whose workspace
+ * (pkv_decode_workspace_bytes) exceeds it returns PKV_E_SCRATCH before any launch. The
  * first call on a device resolves the array's address (make it outside graph capture).
  * Calls on one GPU share the array: calls that overlap on one GPU (concurrent streams)
  * race on it and must be serialised by the caller. Nothing is allocated, copied

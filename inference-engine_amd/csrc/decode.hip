@@ -291,6 +291,17 @@ int check_decode_shape(int kv_dtype, int head_dim, int num_heads, int num_kv_hea
 // address hipGetSymbolAddress returns, kept in g_scratch_ptr.
 static __device__ __align__(256) unsigned char scratch[PKV_NOALLOC_SCRATCH_BYTES];
 
+// The most ranges, num_wg at most, whose scratch fits the static array: the default split's
+// count follows from what the GPU holds at once, and 256 ranges of 128 heads at head_dim 128
+// need 32.5 MiB of records. Whole eights, so that the ranges stay in XCD order. Where not even
+// two ranges fit (the merge plans of a huge batch), num_wg itself, which is then refused.
+int32_t fit_scratch(int32_t num_wg, int32_t batch, int32_t nh, int32_t hd) {
+  int32_t n = num_wg;
+  while (n > 1 && decode_ws(n, batch, nh, hd, false).total > PKV_NOALLOC_SCRATCH_BYTES)
+    n = n > 8 ? (n - 1) / 8 * 8 : n - 1;
+  return n > 1 ? n : num_wg;
+}
+
 constexpr int kMaxDevices = 64;
 void* g_scratch_ptr[kMaxDevices] = {};
 std::mutex g_scratch_mu;
@@ -654,6 +665,10 @@ int pkv_paged_decode_noalloc(void* out, int out_dtype, int64_t out_stride_b,
     sized = pkv_decode_default_workgroups(kv_dtype, head_dim, num_heads, num_kv_heads, batch,
                                           max_blocks, block_size);
     if (sized < 0) return sized;
+  }
+  if (num_workgroups == 0 && sized > 0) {
+    sized = fit_scratch(sized, batch, num_heads, head_dim);
+    num_workgroups = sized;  // the launch takes the count that was sized
   }
   const int64_t need = decode_ws(sized, batch, num_heads, head_dim, false).total;
   if (need > PKV_NOALLOC_SCRATCH_BYTES) return PKV_E_SCRATCH;

@@ -478,8 +478,9 @@ def paged_decode_attention_noalloc(
     is a static per-GPU device array of the library (C ``pkv_paged_decode_noalloc``), the
     result goes to the caller's ``out`` ([B, nh, hd], q.dtype or float32), and q must be
     contiguous. Same kernels and results as ``paged_decode_attention`` at the same
-    ``num_workgroups``. Shapes whose scratch exceeds ``_native.PKV_NOALLOC_SCRATCH_BYTES``
-    raise ValueError; calls that overlap on one GPU (other streams) race on the scratch.
+    ``num_workgroups``. The default split takes at most as many ranges as
+    ``_native.PKV_NOALLOC_SCRATCH_BYTES`` hold; a given count that needs more raises
+    ValueError; calls that overlap on one GPU (other streams) race on the scratch.
     No counterpart in the reference."""
     what = "paged_decode_attention_noalloc"
     dev = _check_decode_args(what, q, k_cache, v_cache, block_tables, context_lens, block_size)

@@ -84,3 +84,27 @@ def test_noalloc_decode_matches_allocating_entry_point():
                                           num_workgroups=1 << 20)  # fmt: skip
     torch.cuda.synchronize()
     assert not out.any()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize(("nh", "nkv", "hd"), [(128, 8, 128), (64, 4, 128), (32, 2, 128), (16, 1, 128),
+                                               (32, 1, 128), (160, 5, 128), (256, 16, 64),
+                                               (64, 8, 128)])  # fmt: skip
+def test_noalloc_default_split_fits_the_scratch(nh, nkv, hd, dtype):
+    """The default split of a batch past the one-launch split pass takes as many ranges as the
+    static array holds: never refused, and the bits of the allocating call at that count."""
+    step = workloads.custom([(7 * i) % 90 for i in range(300)], nh, nkv, hd, 16, dtype, DEV, seed=nh)
+    wgs = pa.default_workgroups(DEV, dtype, hd, nh, nkv, 300, step.block_tables.shape[1], 16)
+    assert wgs > 0
+    size = _native.lib().pkv_decode_workspace_bytes
+    while size(wgs, 300, nh, hd) > _native.PKV_NOALLOC_SCRATCH_BYTES:
+        wgs = (wgs - 1) // 8 * 8
+    _say("noalloc default", nh, nkv, hd, dtype, "ranges", wgs)
+    args = (step.q, step.k_cache, step.v_cache, step.block_tables, step.context_lens, 16)
+    want = torch.empty(step.q.shape, dtype=torch.float32, device=DEV)
+    pa.paged_decode_attention(*args, out=want, num_workgroups=wgs)
+    got = torch.full_like(want, float("nan"))
+    pa.paged_decode_attention_noalloc(*args, out=got)
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)
