@@ -601,52 +601,32 @@ template <> struct Mfma16x16x32<PKV_F16> {
   }
 };
 
-// Four probabilities per lane against four V rows: v_mfma_f32_16x16x16, the contraction
-// of one 16-token tile. P enters as TERMS 16-bit terms, each the rounded rest of the ones
-// before it: bf16 takes three (24 bits, what fp32 P has), fp16 two (22 bits; the caller
-// scales P by 2^7, so weights down to 2^-32 of the largest keep a part).
-template <int DT> struct Mfma16x16x16;
-template <> struct Mfma16x16x16<PKV_BF16> {
-  static constexpr int TERMS = 3;
+// bf16: four probabilities per lane against four V rows, v_mfma_f32_16x16x16, the contraction
+// of one 16-token tile. P enters as three bf16 terms, each the rounded rest of the ones before
+// it: 24 bits over fp32's exponents, what fp32 P has. (fp16's five exponent bits hold no such
+// terms: fp16 takes fp32 MFMAs.)
+struct PTerms {
+  static constexpr int N = 3;
   typedef __bf16 v2 __attribute__((ext_vector_type(2)));
   __device__ static uint32_t pack(float x, float y) {
     return __builtin_bit_cast(uint32_t, v2{(__bf16)x, (__bf16)y});
   }
   __device__ static float low(uint32_t w) { return __uint_as_float(w << 16); }
   __device__ static float high(uint32_t w) { return __uint_as_float(w & 0xFFFF0000u); }
-  __device__ static f32x4 mma(s16x4 a, s16x4 b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0);
-  }
-};
-template <> struct Mfma16x16x16<PKV_F16> {
-  static constexpr int TERMS = 2;
-  typedef _Float16 v2 __attribute__((ext_vector_type(2)));
-  typedef _Float16 v4 __attribute__((ext_vector_type(4)));
-  __device__ static uint32_t pack(float x, float y) {
-    return __builtin_bit_cast(uint32_t, v2{(_Float16)x, (_Float16)y});
-  }
-  __device__ static float low(uint32_t w) { return (float)__builtin_bit_cast(v2, w)[0]; }
-  __device__ static float high(uint32_t w) { return (float)__builtin_bit_cast(v2, w)[1]; }
-  __device__ static f32x4 mma(s16x4 a, s16x4 b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(v4, a),
-                                                 __builtin_bit_cast(v4, b), c, 0, 0, 0);
-  }
-};
-// Probabilities p[0 .. 3] as the terms' operand fragments.
-template <int DT>
-__device__ __forceinline__ void pack_terms(const float* p, s16x4 (&t)[Mfma16x16x16<DT>::TERMS]) {
-  using M = Mfma16x16x16<DT>;
-  float r[4] = {p[0], p[1], p[2], p[3]};
+  s16x4 t[N];
+  __device__ __forceinline__ explicit PTerms(const float* p) {
+    float r[4] = {p[0], p[1], p[2], p[3]};
 #pragma unroll
-  for (int n = 0; n < M::TERMS; ++n) {
-    uint2 w = make_uint2(M::pack(r[0], r[1]), M::pack(r[2], r[3]));
-    // the empty asm keeps the packed pair one value (no second conversion for the rest)
-    __asm__("" : "+v"(w.x), "+v"(w.y));
-    t[n] = __builtin_bit_cast(s16x4, w);
-    r[0] -= M::low(w.x), r[1] -= M::high(w.x);
-    r[2] -= M::low(w.y), r[3] -= M::high(w.y);
+    for (int n = 0; n < N; ++n) {
+      uint2 w = make_uint2(pack(r[0], r[1]), pack(r[2], r[3]));
+      // the empty asm keeps the packed pair one value (no second conversion for the rest)
+      __asm__("" : "+v"(w.x), "+v"(w.y));
+      t[n] = __builtin_bit_cast(s16x4, w);
+      r[0] -= low(w.x), r[1] -= high(w.x);
+      r[2] -= low(w.y), r[3] -= high(w.y);
+    }
   }
-}
+};
 
 __device__ __forceinline__ u32x4 load_kv16v(const void* p) {
 #if PKV_DECODE_STREAM_LOADS
@@ -810,7 +790,6 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeArgs& a, const int 
   const int ng = WIDE ? a.gpw : GPW;  // query heads of this wave
   using S = typename Elt<DT>::S;
   using MMA = Mfma16x16x32<DT>;
-  using MMA4 = Mfma16x16x16<DT>;
   // hd 64: P.V on the matrix cores (PKV_DECODE_PV_MFMA; 5.6% faster than the VALU form,
   // a row broadcast and 8 FMAs per query head and V row, at config 2's batch and
   // contexts; at hd 128, a timing copy without any P.V ran only 1% faster, so it keeps
@@ -822,8 +801,12 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeArgs& a, const int 
   // grp) holds dims 16 d + 4 grp + r.
   // (The stream-K pass only: the split pass's few short steps per wave are latency-bound,
   // and the LDS round trip cost config 1 0.2 us.)
-  // hd 128, wide: the same with one 16-token tile per step (4 KiB of V) and 16x16x16
-  // MFMAs, P in fp32-like terms (pack_terms), as the VALU form it replaces had fp32 P.
+  // hd 128, wide: the same with one 16-token tile per step (4 KiB of V), and P with the bits that
+  // it has in the VALU form: bf16 as three terms (PTerms) on 16x16x16 MFMAs, fp16 as it is, V
+  // widened to fp32, on 16x16x4 fp32 MFMAs. These take four times the matrix time of two fp16
+  // terms (22 bits, and weights below 2^-32 of the reference lost), which the stream pass hides
+  // behind HBM (40 sequences of 800-1,073 tokens, 64 / 8 heads: 40.2 us against 39.6) and the
+  // split pass does not (the same at 32 / 2 heads: 24.9 against 21.2; the VALU form 30.2).
   constexpr bool PVM = pv_mfma<HD, GPW, SPLIT>();
   char* const vslot = reinterpret_cast<char*>(vslots) + (PVM ? (threadIdx.x / kWave) * kVSlotBytes : 0);
 
@@ -1107,11 +1090,11 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeArgs& a, const int 
     constexpr int NACC = PVM ? 1 : GPW, NOV = PVM ? HD / 16 : 1;
     float acc[NACC][8];  // VALU P.V
     f32x4 ov[NOV];       // PVM: O^T, dims 16 d .. 16 d + 15
-    // PVM at hd 128: whether the tiles keep infinities and NaNs of V out of P's lower terms.
+    // PTerms: whether the tiles keep infinities and NaNs of V out of P's lower terms.
     // A term can be 0 where P is not, and 0 x inf would turn an infinite output into NaN: a
     // piece that ends with a NaN runs a second time with them kept out (V is finite in
     // practice, so the first run is free of the checks).
-    constexpr bool kTerms = PVM && NS == 1;
+    constexpr bool kTerms = PVM && NS == 1 && DT == PKV_BF16;
     bool v_careful = false;
 
     // The exponent reference of head column col is raised only when a tile's maximum
@@ -1177,26 +1160,37 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeArgs& a, const int 
         for (int r = 0; r < 4; ++r) p[r] = __builtin_amdgcn_exp2f(p[r] - mref);
         l_run += (p[0] + p[1]) + (p[2] + p[3]);
         if constexpr (PVM) {
-          if constexpr (DT == PKV_F16) {  // scaled as in the hd-64 form below
-#pragma unroll
-            for (int r = 0; r < 4; ++r) p[r] *= 128.f;
-          }
-          s16x4 pt[MMA4::TERMS];
-          pack_terms<DT>(p, pt);
-#pragma unroll
-          for (int d = 0; d < NOV; ++d) ov[d] = MMA4::mma(vt4[d], pt[0], ov[d]);
-          if (v_careful) {  // wave-uniform
-            constexpr short kExp = DT == PKV_BF16 ? 0x7F80 : 0x7C00;
+          if constexpr (kTerms) {
+            const PTerms pt(p);
 #pragma unroll
             for (int d = 0; d < NOV; ++d)
+              ov[d] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(vt4[d], pt.t[0], ov[d], 0, 0, 0);
+            if (v_careful) {  // wave-uniform
+              constexpr short kExp = 0x7F80;
 #pragma unroll
-              for (int e = 0; e < 4; ++e)
-                if ((vt4[d][e] & kExp) == kExp) vt4[d][e] = 0;
+              for (int d = 0; d < NOV; ++d)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                  if ((vt4[d][e] & kExp) == kExp) vt4[d][e] = 0;
+            }
+#pragma unroll
+            for (int n = 1; n < PTerms::N; ++n)
+#pragma unroll
+              for (int d = 0; d < NOV; ++d)
+                ov[d] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(vt4[d], pt.t[n], ov[d], 0, 0, 0);
+          } else {
+            // The tile's sum on its own, then one addition to the running one: a chain of 16
+            // additions to it per tile had 1.15 times the error of the VALU form.
+            f32x4 t[NOV];
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+              for (int d = 0; d < NOV; ++d)
+                t[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                    Elt<DT>::to_f32((uint16_t)vt4[d][j]), p[j], j ? t[d] : f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+            for (int d = 0; d < NOV; ++d) ov[d] += t[d];
           }
-#pragma unroll
-          for (int n = 1; n < MMA4::TERMS; ++n)
-#pragma unroll
-            for (int d = 0; d < NOV; ++d) ov[d] = MMA4::mma(vt4[d], pt[n], ov[d]);
         } else {
         float vf[4][8];
   #pragma unroll
@@ -1356,7 +1350,7 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeArgs& a, const int 
     if constexpr (PVM) {
       // O^T is summed over every token already: lane (head col, grp) holds dims 16 d + 4
       // grp .. + 3 of head h0 + col, and stores them as they are.
-      constexpr float kOScale = DT == PKV_F16 ? 1.f / 128.f : 1.f;  // P's fp16 scale undone
+      constexpr float kOScale = DT == PKV_F16 && HD == 64 ? 1.f / 128.f : 1.f;  // P's fp16 scale undone
       if constexpr (SPLIT) {
         split_merge_wide<DT, HD>(a, b, h0, ng, ov, kOScale, l_tot, m_run, vslots);
         return;

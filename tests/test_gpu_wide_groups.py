@@ -113,3 +113,34 @@ def test_cascade(nkv, hd):
     # the prefix pass is the chunked prefill, whose bar is 2e-3
     assert (outs[1] - outs[0]).abs().max().item() <= 2e-3
     assert (outs[2] - outs[0]).abs().max().item() <= 2e-3
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("group", [4, 8, 16])
+@pytest.mark.parametrize("wgs", [None, 1, 3])
+def test_small_weights_keep_their_bits(group, wgs, dtype):
+    """P is fp32 in P.V at every group size (hd 128): a weight of e^-25 (2^-36) beside one of 1,
+    where the large V is the small weight's, and an infinite V at such a weight. The score -25
+    carries an fp32 rounding of 25 2^-24, which the exponential makes the result's relative
+    error; 2^-18 covers it and the sums."""
+    step = workloads.custom([40, 90], 2 * group, 2, 128, 16, dtype, DEV, seed=5)
+    step.q.zero_()
+    step.q[..., 0] = 16
+    step.k_cache.zero_()
+    step.v_cache.zero_()
+    p = torch.arange(90)
+    for b, n in enumerate([40, 90]):
+        slots = step.block_tables[b].cpu().long()[p[:n] // 16] * 16 + p[:n] % 16
+        step.k_cache[slots.to(DEV), :, 0] = -17.6875  # scores -17.6875 sqrt(2) = -25.01
+        step.k_cache[slots[7], :, 0] = 0
+        step.v_cache[slots[11], :, 3:] = 6e4
+        step.v_cache[slots[n - 3], 0, 1] = float("inf")
+        step.v_cache[slots[n - 3], 1, 2] = float("-inf")
+    out = torch.empty(step.q.shape, dtype=torch.float32, device=DEV)
+    pa.paged_decode_attention(step.q, step.k_cache, step.v_cache, step.block_tables, step.context_lens,
+                              16, out=out, num_workgroups=wgs)  # fmt: skip
+    got, want = out.cpu().double(), _exact(step)
+    assert torch.equal(got.isinf(), want.isinf()) and not got.isnan().any()
+    assert torch.equal(got[want.isinf()], want[want.isinf()])
+    fin = ~want.isinf()
+    assert ((got - want)[fin].abs() <= 2.0**-18 * want[fin].abs()).all()
