@@ -356,6 +356,10 @@ unsigned blocks_for(int64_t n) {
   return (unsigned)(b < 1 ? 1 : (b > 8192 ? 8192 : b));
 }
 
+// Workgroups for kernels that loop over rows, one row (or packet of tokens) per workgroup at a
+// time: HIP launches fewer than 2^32 threads along x.
+unsigned row_grid(int64_t n) { return (unsigned)(n < (1 << 20) ? n : (1 << 20)); }
+
 template <int DX, int DW>
 hipError_t launch_rms(void* out, int64_t so, const void* x, int64_t sx, const RowScale& inv,
                       const void* w, int64_t rows, int cols, hipStream_t st) {
@@ -366,8 +370,7 @@ hipError_t launch_rms(void* out, int64_t so, const void* x, int64_t sx, const Ro
     if (cols % V == 0 && sx % V == 0 && so % V == 0 && aligned16(out) && aligned16(x) &&
         aligned16(w)) {
       const int cvec = cols / V;
-      const unsigned gr = (unsigned)(rows < 0x7FFFFFFF ? rows : 0x7FFFFFFF);
-      hipLaunchKernelGGL((rms_norm_tail_vec_kernel<DX>), dim3(gr), dim3(256), 0, st, (typename F<DX>::S*)out, so,
+      hipLaunchKernelGGL((rms_norm_tail_vec_kernel<DX>), dim3(row_grid(rows)), dim3(256), 0, st, (typename F<DX>::S*)out, so,
                          (const typename F<DX>::S*)x, sx, inv, (const typename F<DX>::S*)w, rows,
                          cvec);
       return hipGetLastError();
@@ -416,7 +419,7 @@ hipError_t launch_rope_hpt(void* x, int64_t sn, int64_t sh, const float* cs, con
   if (items > 0x7FFFFFFF) return hipErrorInvalidValue;
   const int per = items < 256 ? (int)(256 / items) : 1;
   const int64_t wgs = (n + per - 1) / per;
-  hipLaunchKernelGGL((rope_vec_kernel<DT, HPT>), dim3((unsigned)(wgs < 0x7FFFFFFF ? wgs : 0x7FFFFFFF)),
+  hipLaunchKernelGGL((rope_vec_kernel<DT, HPT>), dim3(row_grid(wgs)),
                      dim3(256), 0, st, (typename F<DT>::S*)x, sn, sh, cs, sn_, sc, n, heads, half,
                      (int)items, per);
   return hipGetLastError();

@@ -88,3 +88,13 @@ def test_silu_mul_streamed(dtype):
         g, u = (torch.randn(m, device=DEV).to(dtype) for _ in range(2))
         g[-3], u[5] = float("nan"), float("inf")
         assert _same(fused.silu_mul(g, u), F.silu(g) * u)
+
+
+def test_rms_norm_more_rows_than_a_grid_holds():
+    """2^24 workgroups of 256 threads are past HIP's 2^32 threads along x."""
+    rows = (1 << 24) + 3
+    x = torch.randn(rows, 8, device=DEV).bfloat16()
+    w = torch.randn(8, device=DEV).bfloat16()
+    got = fused.rms_norm(x, w, 1e-5)
+    for lo in range(0, rows, 1 << 22):
+        assert _same(got[lo : lo + (1 << 22)], _rms(x[lo : lo + (1 << 22)], w, 1e-5))
