@@ -98,3 +98,22 @@ def test_rms_norm_more_rows_than_a_grid_holds():
     got = fused.rms_norm(x, w, 1e-5)
     for lo in range(0, rows, 1 << 22):
         assert _same(got[lo : lo + (1 << 22)], _rms(x[lo : lo + (1 << 22)], w, 1e-5))
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("cols", [1, 3, 4, 8, 12, 33, 64, 72, 128, 256, 264, 511, 512, 520, 1032])
+@pytest.mark.parametrize("rows", [1, 7, 2053])
+def test_rms_norm_several_rows_per_workgroup(rows, cols, dtype):
+    """Rows of 1 to 64 vectors share workgroups, in both widths of access; the last workgroup is
+    partly filled. 65,535 workgroups along y and a row more go round the loop."""
+    x = torch.randn(rows, cols + 8, device=DEV).to(dtype)[:, :cols]
+    w = torch.randn(cols, device=DEV).to(dtype)
+    assert _same(fused.rms_norm(x, w, 1e-5), _rms(x, w, 1e-5))
+    w32 = w.float()  # another weight dtype: one element per access
+    assert _same(fused.rms_norm(x, w32, 1e-5), _rms(x, w32, 1e-5))
+
+
+def test_rms_norm_rows_past_the_grid():
+    x = torch.randn(65535 * 4 + 5, 33, device=DEV)
+    w = torch.randn(33, device=DEV)
+    assert _same(fused.rms_norm(x, w, 1e-5), _rms(x, w, 1e-5))
