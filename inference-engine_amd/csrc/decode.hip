@@ -88,7 +88,7 @@ template <int DT, int HD, int GPW> const void* decode_kernel() {
     return reinterpret_cast<const void*>(
         &paged_decode_mfma_kernel<DT, stream_gpw<HD, GPW>(), true, HD, false>);
   else
-    return reinterpret_cast<const void*>(&paged_decode_stream_kernel<DT, HD, GPW>);
+    return reinterpret_cast<const void*>(&paged_decode_stream_kernel<DT, HD, GPW, false>);
 }
 
 // Dynamic LDS of the stream pass's workgroups of wpg waves.
@@ -165,8 +165,10 @@ struct LaunchDecode {
       } else {
         launch_stream<DT, HD, GPW, false>(grid, block, lds, staged);
       }
+    } else if (a->rows) {
+      hipLaunchKernelGGL((paged_decode_stream_kernel<DT, HD, GPW, true>), grid, block, 0, st, *a);
     } else {
-      hipLaunchKernelGGL((paged_decode_stream_kernel<DT, HD, GPW>), grid, block, 0, st, *a);
+      hipLaunchKernelGGL((paged_decode_stream_kernel<DT, HD, GPW, false>), grid, block, 0, st, *a);
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || (a->num_wg <= 1 && !a->pre_row)) return e;

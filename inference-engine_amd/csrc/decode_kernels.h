@@ -343,7 +343,10 @@ __device__ __forceinline__ int staged_owner(const DecodeArgs& a, const BatchLds&
   return lo;
 }
 
-template <int DT, int HD, int GPW>
+// ROWS: a.rows may be non-null. A form of its own: with the lookup at run time the plain one took 2
+// registers more (fp32 at head_dim 64, 4 heads: 173, a wave per SIMD less), and 64 sequences of
+// 100-919 tokens, 16 / 2 heads, hd 256, bf16 38.7 us against 37.0.
+template <int DT, int HD, int GPW, bool ROWS>
 __global__ void __launch_bounds__(512)
 paged_decode_stream_kernel(const DecodeArgs a) {
   using Sh = DecodeShape<DT, HD>;
@@ -380,7 +383,7 @@ paged_decode_stream_kernel(const DecodeArgs a) {
     ub = ue;
 
     // Query rows of this wave for sequence b, pre-scaled into the exp2 domain.
-    const int64_t srow = seq_row(a, b);
+    const int64_t srow = ROWS ? seq_row(a, b) : b;
     float qf[GPW][VEC];
 #pragma unroll
     for (int g = 0; g < GPW; ++g) {
@@ -513,7 +516,9 @@ paged_decode_stream_kernel(const DecodeArgs a) {
 
     if (lane < LPT) {
       if (whole) {  // the whole context was in this range: final output directly
-        if (srow < 0) continue;
+        if constexpr (ROWS) {
+          if (srow < 0) continue;
+        }
         const WholeDst dst = whole_dst(a, pre_b);
 #pragma unroll
         for (int g = 0; g < GPW; ++g) {

@@ -111,3 +111,11 @@ def test_rows_outside_are_skipped():
         assert (out[[0, 2, 3]] == 7).all() and not (out[1] == 7).any()
     with pytest.raises(ValueError, match="rows"):
         pa.paged_decode_attention(q, *args, rows=rows)
+
+
+@pytest.mark.gpu
+def test_plain_decode_keeps_its_registers():
+    """The row lookup is a form of its own: in the plain one it cost registers, and fp32 at hd 64
+    (4 heads per wave: 168 of them) a wave per SIMD, 2 workgroups of 4 waves per CU for 3."""
+    cus = torch.cuda.get_device_properties(DEV).multi_processor_count
+    assert pa.decode_workgroups(DEV, torch.float32, 64, 16, 4) == 3 * cus
