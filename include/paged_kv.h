@@ -100,7 +100,8 @@ int32_t pkv_decode_workgroups(int kv_dtype, int32_t head_dim, int32_t num_heads,
 /*
  * What num_workgroups = 0 (the default split) of pkv_paged_decode runs for this shape
  * without cascade extras: 0 for the one-kernel split pass (no workspace), else the
- * stream-K workgroup count (pkv_decode_workgroups), whose workspace the caller passes.
+ * stream-K workgroup count (at most pkv_decode_workgroups; fewer for groups of 5 to 16 heads
+ * and short batches), whose workspace the caller passes.
  * Depends on static shapes and the device only. Negative: a PKV_E_* code.
  */
 int32_t pkv_decode_default_workgroups(int kv_dtype, int32_t head_dim, int32_t num_heads,
@@ -135,7 +136,7 @@ int64_t pkv_decode_workspace_bytes(int32_t num_workgroups, int32_t batch, int32_
  * run one kernel with one workgroup per (sequence, KV head, sub-group of its query
  * heads -- as few heads, 16 at most, as keep the workgroups within the CUs) that splits the
  * sequence among its waves and merges in LDS (no workspace used); everything else the
- * split above with pkv_decode_workgroups() workgroups, whose workspace size the caller
+ * split above with pkv_decode_default_workgroups() workgroups, whose workspace size the caller
  * passes.
  */
 int pkv_paged_decode(void* out, int out_dtype, int64_t out_stride_b, int64_t out_stride_h,

@@ -6,6 +6,7 @@
 #include "cascade.h"
 #include "decode_kernels.h"
 
+#include <algorithm>
 #include <mutex>
 
 namespace {
@@ -266,6 +267,26 @@ DecodePlan plan_cascade(int kv_dtype, int head_dim, int num_heads, int num_kv_he
   return n.wpg == PKV_DECODE_WAVES_PER_WG ? n : p;
 }
 
+constexpr int kMaxDevices = 64;
+
+// CU count of the current device, queried once per device.
+int g_cus[kMaxDevices] = {};
+std::mutex g_cus_mu;
+int device_cus(int* cus) {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return PKV_E_HIP;
+  std::lock_guard<std::mutex> lock(g_cus_mu);
+  if (!g_cus[dev]) {
+    int n = 0;
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+        n < 1)
+      return PKV_E_HIP;
+    g_cus[dev] = n;
+  }
+  *cus = g_cus[dev];
+  return 0;
+}
+
 // Workgroups of a plan that the current device holds at once (see pkv_decode_workgroups).
 int32_t plan_workgroups(const DecodePlan& p, int kv_dtype, int head_dim) {
   int dev = 0, cus = 0, per_cu = 0, tile = 0;
@@ -275,6 +296,32 @@ int32_t plan_workgroups(const DecodePlan& p, int kv_dtype, int head_dim) {
   if (e != hipSuccess) return PKV_E_HIP;
   const int g = cus * (per_cu < 1 ? 1 : per_cu) / p.ygrid;
   return g < 1 ? 1 : g;
+}
+
+// Ranges of the default stream-K split of a batch whose tables hold `max_tokens` tokens: what the
+// device holds at once, but for the wide form, whose ranges cost more (a record of up to 16 heads
+// for each, folded by the combine). There (us per call at this many ranges):
+//   * four waves per CU where the ranges would hold fewer than 24 tiles of 16 tokens: 16 / 1
+//     heads, 64 sequences of 100-3,943 tokens, 2,048 / 1,024 ranges 30.1 / 27.6; 32 / 2, 1,024 /
+//     512 39.8 / 37.4; but 130 of 100-3,841, fp16 (30 tiles), 63.0 / 74.6;
+//   * past one workgroup per CU, at least gpw / 2 tiles per range: its records are then a quarter
+//     of the K/V it reads (64 / 4, one sequence of 20,011 tokens, 512 / 256 ranges 31.4 / 23.5;
+//     8 / 1, 300 of 20-99, 2,048 / 1,024 / 512 20.7 / 16.5 / 15.9);
+//   * up to there, at least gpw / 4, down to 64 ranges: 128 / 8, one sequence of 2,500, 256 / 128
+//     / 64 21.7 / 18.6 / 17.5 (18.2 in waves of 4 heads); of 8,000, 256 / 128 / 64 27.1 / 24.2 /
+//     27.2; 64 / 8, of 8,000, 256 / 128 21.6 / 20.7.
+int32_t default_ranges(const DecodePlan& p, int kv_dtype, int head_dim, int batch, int64_t max_tokens) {
+  const int32_t full = plan_workgroups(p, kv_dtype, head_dim);
+  if (p.gpw <= 4 || full < 1) return full;
+  int cus = 0;
+  const int st = device_cus(&cus);
+  if (st) return st;
+  const int64_t tiles = (int64_t)batch * ((max_tokens + 15) / 16);
+  int64_t r = full;
+  if (tiles < 24 * r) r = std::min<int64_t>(r, (int64_t)cus * ((p.wpg + 3) / p.wpg));
+  if (r > cus) r = std::max<int64_t>(cus, std::min(r, tiles * 2 / p.gpw / cus * cus));
+  if (r <= cus) r = std::max(std::min<int64_t>(r, 64), std::min(r, (tiles * 4 / p.gpw + 7) / 8 * 8));
+  return (int32_t)r;
 }
 
 int check_decode_shape(int kv_dtype, int head_dim, int num_heads, int num_kv_heads) {
@@ -304,27 +351,8 @@ int32_t fit_scratch(int32_t num_wg, int32_t batch, int32_t nh, int32_t hd) {
   return n > 1 ? n : num_wg;
 }
 
-constexpr int kMaxDevices = 64;
 void* g_scratch_ptr[kMaxDevices] = {};
 std::mutex g_scratch_mu;
-
-// CU count of the current device, queried once per device.
-int g_cus[kMaxDevices] = {};
-std::mutex g_cus_mu;
-int device_cus(int* cus) {
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return PKV_E_HIP;
-  std::lock_guard<std::mutex> lock(g_cus_mu);
-  if (!g_cus[dev]) {
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        n < 1)
-      return PKV_E_HIP;
-    g_cus[dev] = n;
-  }
-  *cus = g_cus[dev];
-  return 0;
-}
 
 // Whether a default-split call (num_workgroups == 0) takes the per-sequence split pass,
 // and with how many query heads per wave (*gpw, 0 = no): 16-bit K/V at head_dim 64 or
@@ -422,7 +450,11 @@ int decode_ex(void* out, int out_dtype, int64_t out_stride_b, int64_t out_stride
       p.gpw = split_gpw;
       p.nsub = num_heads / num_kv_heads / split_gpw;
     } else {
-      num_workgroups = plan_workgroups(p, kv_dtype, head_dim);
+      // A cascade's workspace is sized by what the device holds (its callers ask
+      // pkv_decode_workgroups).
+      num_workgroups = cascade ? plan_workgroups(p, kv_dtype, head_dim)
+                               : default_ranges(p, kv_dtype, head_dim, batch,
+                                                (int64_t)max_blocks * block_size);
       if (num_workgroups < 1) return num_workgroups < 0 ? num_workgroups : PKV_E_HIP;
     }
   }
@@ -576,7 +608,9 @@ int32_t pkv_decode_default_workgroups(int kv_dtype, int32_t head_dim, int32_t nu
   const int st = choose_split(kv_dtype, head_dim, batch, num_heads, num_kv_heads, max_blocks,
                               (int64_t)max_blocks * block_size, false, &split_gpw);
   if (st) return st;
-  return split_gpw ? 0 : pkv_decode_workgroups(kv_dtype, head_dim, num_heads, num_kv_heads);
+  if (split_gpw) return 0;
+  return default_ranges(plan_decode(kv_dtype, head_dim, num_heads, num_kv_heads), kv_dtype, head_dim,
+                        batch, (int64_t)max_blocks * block_size);
 }
 
 int64_t pkv_decode_workspace_bytes(int32_t num_workgroups, int32_t batch, int32_t num_heads,

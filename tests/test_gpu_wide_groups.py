@@ -144,3 +144,22 @@ def test_small_weights_keep_their_bits(group, wgs, dtype):
     assert torch.equal(got[want.isinf()], want[want.isinf()])
     fin = ~want.isinf()
     assert ((got - want)[fin].abs() <= 2.0**-18 * want[fin].abs()).all()
+
+
+@pytest.mark.parametrize(("nh", "nkv", "ctx", "most"), [
+    (128, 8, [2500], 64), (128, 8, [8000], 128), (64, 4, [20011], 256), (32, 2, [3000, 2800, 3300, 2900], 256),
+    (16, 1, [20 + i % 80 for i in range(300)], 256), (8, 1, [20 + i % 80 for i in range(300)], 512),
+    (16, 1, [1000 + i for i in range(300)], 1024), (32, 2, [300 + i for i in range(300)], 512), (40, 8, [300 + i for i in range(40)], 256),
+    (15, 3, [2000 + i for i in range(300)], 512), (160, 16, [2500], 64)])  # fmt: skip
+def test_default_ranges(nh, nkv, ctx, most):
+    """The default split of the wide form cuts short batches into fewer ranges than the GPU holds:
+    a range's records are a fraction of the K/V it reads."""
+    step = workloads.custom(ctx, nh, nkv, 128, 16, torch.bfloat16, DEV, seed=2)
+    wgs = pa.default_workgroups(DEV, torch.bfloat16, 128, nh, nkv, len(ctx), step.block_tables.shape[1], 16)
+    cus = torch.cuda.get_device_properties(DEV).multi_processor_count
+    print("[case] ranges", nh, nkv, len(ctx), wgs, flush=True)
+    assert 32 <= wgs <= pa.decode_workgroups(DEV, torch.bfloat16, 128, nh, nkv)
+    if cus == 256:
+        assert wgs <= most
+    if len(ctx) < 300:
+        _check(step)
