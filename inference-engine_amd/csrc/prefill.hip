@@ -64,7 +64,9 @@ paged_prefill_f32_kernel(const PrefillArgs a) {
   const int lane = tid & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(htid / kWave);
   const int col = lane & 15, grp = lane >> 4;
-  const PrefillItem it = pick_item(a, (int)blockIdx.x);
+  const unsigned item = blockIdx.y * gridDim.x + blockIdx.x;
+  if (item >= (unsigned)(a.row_blocks * a.nkv * a.n_chunks)) return;  // of < 2^31 items
+  const PrefillItem it = pick_item(a, (int)item);
   const int c = it.c, q0 = it.q0, n = it.n, kvh = it.kvh;
   const int qlen = it.q1 - q0, G = a.groups, nrows = qlen * G;
   const int rho0 = (a.row_blocks - 1 - it.rbi) * BM;
@@ -298,12 +300,16 @@ hipError_t launch_v16(const PrefillArgs& a, int hd, hipStream_t st) {
   return hipGetLastError();
 }
 
-// The fp32 kernel: one workgroup per item (chunk, 64-row block, KV head).
+// The fp32 kernel: one workgroup per item (chunk, 64-row block, KV head). On two grid dimensions:
+// a bound on the chunks' lengths that few of them reach makes many empty items, and HIP launches
+// fewer than 2^32 threads along x.
 template <int DT, int HD> hipError_t launch_f32_hd(PrefillArgs a, int64_t rows, hipStream_t st) {
   a.row_blocks = (int)((rows + F32Shape<HD>::BM - 1) / F32Shape<HD>::BM);
   const int64_t items = (int64_t)a.row_blocks * a.nkv * a.n_chunks;
   if (items > 0x7FFFFFFF) return hipErrorInvalidValue;
-  hipLaunchKernelGGL((paged_prefill_f32_kernel<DT, HD>), dim3((unsigned)items), dim3(512), 0, st, a);
+  const int64_t gx = items < (1 << 20) ? items : (1 << 20);
+  hipLaunchKernelGGL((paged_prefill_f32_kernel<DT, HD>),
+                     dim3((unsigned)gx, (unsigned)((items + gx - 1) / gx)), dim3(512), 0, st, a);
   return hipGetLastError();
 }
 hipError_t launch_f32(const PrefillArgs& a, int hd, int64_t rows, hipStream_t st) {

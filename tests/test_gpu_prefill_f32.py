@@ -55,3 +55,14 @@ def test_tile_edges(nh, nkv, bs, hd, dtype):
     err = (out.cpu().double() - _exact(step, lens)).abs().max().item()
     assert err <= TOL, err
     assert torch.equal(rounded, out.to(dtype))
+
+
+def test_more_items_than_one_grid_dimension_holds():
+    """A bound on the chunks' lengths far above them: 2,100 x 512 x 8 items of 512 threads, past
+    HIP's 2^32 along x; nearly all of them empty."""
+    lens = [1 + i % 3 for i in range(2100)]
+    step = workloads.custom([n + i % 40 for i, n in enumerate(lens)], 8, 8, 16, 16, torch.float32, DEV, seed=1)
+    q = torch.randn(sum(lens), 8, 16, device=DEV)
+    cu = torch.tensor([0, *torch.tensor(lens).cumsum(0).tolist()], dtype=torch.int32, device=DEV)
+    args = (q, step.k_cache, step.v_cache, step.block_tables, step.context_lens, 16, cu)
+    assert torch.equal(pa.paged_prefill_attention(*args, 32768), pa.paged_prefill_attention(*args, 3))
