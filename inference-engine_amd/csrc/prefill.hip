@@ -232,24 +232,100 @@ paged_prefill_f32_kernel(const PrefillArgs a) {
       for (int r = 0; r < 4; ++r) x[(4 * d + r) * kWave] = ov[d][r];
   }
   __syncthreads();
-  if (half || !row_ok) return;
+  if (half) return;
   const float mb = xml[wave][0][lane];
   const float mn = fmaxf(m_run, mb);
   const float mref = mn == -INFINITY ? 0.f : mn;  // both empty: weights 0
   const float sa = __builtin_amdgcn_exp2f(m_run - mref), sb = __builtin_amdgcn_exp2f(mb - mref);
   l_tot = l_tot * sa + xml[wave][1][lane] * sb;
   const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;  // nothing visible: 0
-  const int64_t e0 = orow * a.out_st + (int64_t)head * a.out_sh + 4 * grp;
+  const int64_t e0 = orow * a.out_st + (int64_t)head * a.out_sh;
+  bool nan = false;
 #pragma unroll
   for (int d = 0; d < DTL; ++d) {
     float o[4];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) o[r] = (ov[d][r] * sa + x[(4 * d + r) * kWave] * sb) * inv;
-    if (a.out_f32) store_vec<PKV_F32, 4>((float*)a.out + e0 + 16 * d, o);
-    else store_vec<DT, 4>((S*)a.out + e0 + 16 * d, o);
+    for (int r = 0; r < 4; ++r) {
+      o[r] = (ov[d][r] * sa + x[(4 * d + r) * kWave] * sb) * inv;
+      nan = nan || o[r] != o[r];
+    }
+    if (!row_ok) continue;
+    if (a.out_f32) store_vec<PKV_F32, 4>((float*)a.out + e0 + 16 * d + 4 * grp, o);
+    else store_vec<DT, 4>((S*)a.out + e0 + 16 * d + 4 * grp, o);
   }
-  if (a.lse && grp == 0)
+  if (a.lse && row_ok && grp == 0)
     a.lse[(int64_t)(q0 + tok) * a.nh + head] = l_tot > 0.f ? mn + __log2f(l_tot) : -INFINITY;
+
+  // Keys past a row's last one enter its P.V with P = 0, and 0 x inf is NaN: a row that holds a NaN,
+  // with an infinite or NaN V among those keys of its tiles, is computed again without them, by the
+  // whole wave, 64 keys at a time. Rare (V is finite in practice), so it is only kept small.
+  uint64_t redo = __ballot(nan && row_ok);
+  redo = (redo | redo >> 16 | redo >> 32 | redo >> 48) & 0xFFFF;
+  const int kused = min(kend, (wlimit / TK + 1) * TK);
+  const S* kb = reinterpret_cast<const S*>(a.k) + (int64_t)kvh * a.kv_sh;
+  const S* vb = reinterpret_cast<const S*>(a.v) + (int64_t)kvh * a.kv_sh;
+  auto slot_of = [&](int p, int last) -> int64_t {  // key p's slot, -1 past `last` or the pool
+    if (p > last) return -1;
+    const int blk = blk_of(p), id = trow[blk];
+    const int64_t sl = (int64_t)id * a.bs + (p - blk * a.bs);
+    return id >= 0 && sl < a.num_slots ? sl : -1;
+  };
+  for (; redo; redo &= redo - 1) {
+    const int row = __builtin_ctzll(redo);  // lane `row` holds it (and + 16, 32, 48)
+    const int last = __builtin_amdgcn_readlane(limit, row);
+    bool bad = false;
+    for (int p = last + 1 + lane; p < kused; p += kWave) {
+      const int64_t sl = slot_of(p, kused);
+      for (int e = 0; sl >= 0 && e < HD; ++e) {
+        const float v = Elt<DT>::to_f32(vb[sl * a.kv_ss + e]);
+        bad = bad || !(fabsf(v) < INFINITY);
+      }
+    }
+    if (!__ballot(bad)) continue;
+    auto score = [&](int64_t sl) {
+      float sc1 = 0.f;
+#pragma unroll
+      for (int i = 0; i < HD / 16; ++i) {
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const float qv = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(qf[i][j]), row + 16 * g));
+            sc1 = __builtin_fmaf(qv, Elt<DT>::to_f32(kb[max(sl, (int64_t)0) * a.kv_ss + 16 * i + 4 * g + j]), sc1);
+          }
+        __builtin_amdgcn_sched_barrier(0);  // few loads in flight: few registers
+      }
+      return sl >= 0 ? sc1 : -INFINITY;
+    };
+    float mr = -INFINITY, lr = 0.f, acc[(HD + kWave - 1) / kWave] = {};
+    for (int p = 0; p <= last; p += kWave) mr = fmaxf(mr, score(slot_of(p + lane, last)));
+#pragma unroll
+    for (int off = 1; off < kWave; off <<= 1) mr = fmaxf(mr, __shfl_xor(mr, off));
+    for (int p = 0; p <= last; p += kWave) {
+      const int64_t sl = slot_of(p + lane, last);
+      const float pr = __builtin_amdgcn_exp2f(score(sl) - (mr == -INFINITY ? 0.f : mr));
+      lr += pr;
+      for (int t = 0; t < kWave && p + t <= last; ++t) {
+        const int64_t st = __shfl(sl, t);
+        const float pt = __shfl(pr, t);
+#pragma unroll
+        for (int k = 0; k < (HD + kWave - 1) / kWave; ++k)
+          if (st >= 0 && lane + kWave * k < HD)
+            acc[k] = __builtin_fmaf(pt, Elt<DT>::to_f32(vb[st * a.kv_ss + lane + kWave * k]), acc[k]);
+      }
+    }
+#pragma unroll
+    for (int off = 1; off < kWave; off <<= 1) lr += __shfl_xor(lr, off);
+    const float invr = lr > 0.f ? 1.f / lr : 0.f;
+    const int64_t er = __shfl(e0, row);
+#pragma unroll
+    for (int k = 0; k < (HD + kWave - 1) / kWave; ++k) {
+      const int d = lane + kWave * k;
+      if (d >= HD) break;
+      if (a.out_f32) reinterpret_cast<float*>(a.out)[er + d] = acc[k] * invr;
+      else reinterpret_cast<S*>(a.out)[er + d] = Elt<DT>::from_f32(acc[k] * invr);
+    }
+  }
 }
 
 // ---------------------------------------------------------------------------------

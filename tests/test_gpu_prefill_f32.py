@@ -66,3 +66,32 @@ def test_more_items_than_one_grid_dimension_holds():
     cu = torch.tensor([0, *torch.tensor(lens).cumsum(0).tolist()], dtype=torch.int32, device=DEV)
     args = (q, step.k_cache, step.v_cache, step.block_tables, step.context_lens, 16, cu)
     assert torch.equal(pa.paged_prefill_attention(*args, 32768), pa.paged_prefill_attention(*args, 3))
+
+
+@pytest.mark.parametrize(("hd", "dtype"), [(16, torch.float32), (16, torch.bfloat16), (64, torch.float32),
+                                           (128, torch.float32), (256, torch.float32)])  # fmt: skip
+@pytest.mark.parametrize("groups", [1, 2, 3, 8])
+@pytest.mark.parametrize("value", [float("inf"), float("nan")])
+def test_later_values_do_not_reach_earlier_rows(groups, hd, dtype, value):
+    """An infinite or NaN V of a token shows in its own row and the later ones of its chunk, in its
+    dim, and nowhere else (an earlier row's P is 0 there, and 0 x inf is NaN): also where out is q."""
+    lens, cached = [90, 33], [37, 0]
+    step = workloads.custom([127, 33], 2 * groups, 2, hd, 16, dtype, DEV, seed=hd)
+    q = torch.randn(sum(lens), 2 * groups, hd, device=DEV).to(dtype)
+    step.info["q"] = q
+    cu = torch.tensor([0, 90, 123], dtype=torch.int32, device=DEV)
+    want = _exact(step, lens)
+    for c, t in ((0, 40), (0, 89), (1, 20)):  # token t of chunk c
+        p = cached[c] + t
+        step.v_cache[int(step.block_tables[c, p // 16]) * 16 + p % 16, :, hd // 2] = value
+    args = (step.k_cache, step.v_cache, step.block_tables, step.context_lens, 16, cu, 90)
+    out = torch.empty(q.shape, device=DEV)
+    rounded = q.clone()
+    pa.paged_prefill_attention(q, *args, out=out)
+    pa.paged_prefill_attention(rounded, *args, out=rounded, rows=torch.arange(123, device=DEV))
+    assert torch.equal(rounded.nan_to_num(7.0), out.to(dtype).nan_to_num(7.0))
+    out = out.cpu().double()
+    hit = torch.zeros(out.shape, dtype=torch.bool)
+    hit[[*range(40, 90), *range(110, 123)], :, hd // 2] = True
+    assert (out[~hit] - want[~hit]).abs().max().item() <= TOL
+    assert (out[hit].isnan() if value != value else out[hit] == value).all()
