@@ -359,7 +359,7 @@ template <int HD> struct PrefillLds {
 };
 
 // One work item on a workgroup of 512 threads. V16: P.V in fp16 with V from the fp16
-// copy. Every exit is workgroup-uniform except half 1's after the merge; a caller that
+// copy (bf16 caches; the launch guarantees every chunk's region). Every exit is workgroup-uniform except half 1's after the merge; a caller that
 // runs several items on one workgroup puts a barrier between them (the merge reuses the
 // rings).
 // ROWS: q and out rows through a.rows (else a.rows is null).
@@ -1108,17 +1108,13 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs& a, const Prefill
   }
 }
 
-// One work item (chunk, 128-row block, KV head) on a workgroup of 512 threads. Every
-// exit is workgroup-uniform except half 1's after the merge; a caller that runs several
-// items on one workgroup puts a barrier between them (the merge reuses the rings).
-// V16: V from the fp16 copy (bf16 caches; the launch guarantees every chunk's region).
 // The coordinates of item `item`.
 __device__ __forceinline__ PrefillItem pick_item(const PrefillArgs& a, const int item) {
   const int lane = threadIdx.x & (kWave - 1);
   // Work items (chunk, row block, KV head), heaviest first: chunks by context length
   // (longest first), then row blocks from the last (it sees the most keys), KV heads
-  // innermost. One workgroup fills a CU, so a grid larger than the GPU runs the items
-  // in this order as CUs free up: the longest start earliest.
+  // innermost. A grid larger than the GPU holds at once runs the items in this order as
+  // CUs free up: the longest start earliest.
   PrefillItem it;
   it.kvh = item % a.nkv;
   it.rbi = (item / a.nkv) % a.row_blocks;
@@ -1149,6 +1145,7 @@ __device__ __forceinline__ PrefillItem pick_item(const PrefillArgs& a, const int
   return it;
 }
 
+// Item `item` (chunk, row block, KV head): prefill_body at its coordinates.
 template <int DT, int HD, bool POW2, bool V16, bool ROWS>
 __device__ __forceinline__ void prefill_item(const PrefillArgs& a, const int item,
                                              PrefillLds<HD>& lds) {
@@ -1156,10 +1153,12 @@ __device__ __forceinline__ void prefill_item(const PrefillArgs& a, const int ite
 }
 
 // Head_dim 32 and 64 leave room for two workgroups on a CU (72 KB of LDS each at 64): the
-// kernels whose registers fit 128 without spilling are held to that (bf16 with the copy of
-// V at head_dim 64 took 131 and ran one workgroup per CU: 12 ragged chunks of 3-600 tokens
-// behind up to 3,000 cached ones, 32 / 8 heads, 109.6 us per call, now 90.4; bf16 without the
-// copy would spill 18).
+// kernels whose registers fit 128 are held to that (bf16 with the copy of V at head_dim 64 took
+// 131 and ran one workgroup per CU: 12 ragged chunks of 3-600 tokens behind up to 3,000 cached
+// ones, 32 / 8 heads, 109.6 us per call, now 90.4; bf16 without the copy would spill 18). One of
+// them spills: fp16 at head_dim 64 with ROWS, 2 registers that the loop does not use. Looking
+// the rows of out up again at the end frees them and is not faster (76.3 us against 75.9 on
+// such chunks; at head_dim 128, where nothing spills, 131.7 against 129.4).
 template <int DT, int HD, bool V16> constexpr bool prefill_two_wgs() {
   return HD <= 64 && (DT != PKV_BF16 || V16);
 }
