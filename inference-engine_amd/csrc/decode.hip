@@ -108,14 +108,18 @@ template <int DT, int HD, int GPW> constexpr unsigned stream_lds(int wpg) {
 //   1,024 pairs (64 of 200-3,000, 16 heads)         71.3 / 71.4 / 72.1 / 74.6 / 77.9
 //   1,024 pairs (32 of 128-32,768, log)            106.9 / 105.7 / 105.0 / 106.5 / 110.1
 //   1,536 pairs (64 of 1,024-4,096, 24 heads)      109.8 / 110.0 / 111.6 / 115.0 / 119.8
-// At 1,024 pairs four waves pay where sequences have many pieces (8 or more ranges each).
+//   768 pairs (24 of 3,000-9,000, 24 heads)        103.4 / 101.8 / 104.2 / 105.3 / 112.0
+//   1,024 pairs (32 of 2,060-2,200)                 56.9 / 54.5 / 56.1 / 57.2 / 64.4
+//   32 pairs, hd 256 (1 of 20,011)                  65.6 / 54.0 / 47.0 / 44.4 / 44.4
+//   8 pairs, hd 256 (1 of 9,000, 8 heads)          122.2 / 74.6 / 43.8 / 34.0 / 30.3
+// (Four waves up to 1,024 pairs gain 0.5-1% where a few long sequences have most of the ranges, 32
+// of 128-32,768, and lose 1-3% elsewhere.)
 int combine_waves(const DecodeArgs& a) {
   const int pairs = a.batch * a.nh;
   if (pairs <= 64) return 16;
   if (pairs <= 256) return 8;
   if (pairs <= 512) return 4;
-  if (pairs > PKV_DECODE_COMBINE_SPLIT_PAIRS) return 1;
-  return a.num_wg >= 8 * a.batch ? 4 : 2;
+  return pairs <= PKV_DECODE_COMBINE_SPLIT_PAIRS ? 2 : 1;
 }
 template <int DT, int HD, int SP, bool WT, bool ROWS>
 void launch_combine_sp(const DecodeArgs& a, hipStream_t st) {
