@@ -57,6 +57,10 @@ def mixed_attention(layer_idx: int, q: torch.Tensor, batch: PagedBatch,
     if batch.chunks:
         raise ValueError("mixed_attention: per-chunk SDPA entries (PagedBatch.chunks) "
                          "belong to the reference's gather path")  # fmt: skip
+    if min(q.shape[0], q.shape[0] if out is None else out.shape[0]) < batch.num_tokens:
+        # the kernels skip rows that q does not have, where indexing raises
+        raise IndexError(f"mixed_attention: a step of {batch.num_tokens} tokens on q {tuple(q.shape)}"
+                         + (f", out {tuple(out.shape)}" if out is not None else ""))  # fmt: skip
     cache = batch.cache
     kc, vc, bs = cache.k[layer_idx], cache.v[layer_idx], cache.block_size
     if out is None:

@@ -275,7 +275,7 @@ class MixedGraphs:
             last_index=self._last, use_kernel=False, mixed=True, decode_rows=self._dec_rows,
             block_tables=self._dec_tab, context_lens=self._dec_ctx, chunks=[],
             chunk_rows=self._ch_rows[:n], chunk_tables=self._ch_tab, chunk_ctx=self._ch_ctx,
-            cu_seqlens_q=self._cu_q, max_query_len=n)  # fmt: skip
+            cu_seqlens_q=self._cu_q, max_query_len=n, num_tokens=n)  # fmt: skip
 
     def _forward(self, n: int) -> torch.Tensor:
         return self.model(self._ids[:, :n], self._pos[:, :n], self._views[n])

@@ -226,6 +226,8 @@ class PagedBatch:
     # Decode steps with cascade on: the groups of sequences sharing leading blocks
     # (engine.kernels.paged_attention.PrefixGroups), or None.
     prefix_groups: object | None = None
+    # Mixed steps: the rows of q and out that decode_rows and chunk_rows index (0: not known).
+    num_tokens: int = 0
 
     @classmethod
     def build(
@@ -379,7 +381,7 @@ class PagedBatch:
                     q_valid=torch.zeros(0, dtype=torch.bool, device=device), attn_mask=None,
                     last_index=torch.cumsum(qlens, 0) - 1, use_kernel=False, mixed=True,
                     decode_rows=torch.tensor(dec_rows, dtype=torch.int64, device=device),
-                    chunks=[])  # fmt: skip
+                    chunks=[], num_tokens=start)  # fmt: skip
         if dec_rows:
             batch.block_tables = cls._tables(dec_tables).to(device)
             batch.context_lens = torch.tensor(dec_ctx, dtype=torch.int32, device=device)

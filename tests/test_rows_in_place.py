@@ -8,6 +8,8 @@ import torch
 
 from engine import workloads
 from engine.kernels import paged_attention as pa
+from engine.model.layers import mixed_attention
+from engine.runtime.paged_cache import KVShape, PagedBatch, PagedKVCache
 
 DEV = torch.device("cuda:0")
 
@@ -119,3 +121,16 @@ def test_plain_decode_keeps_its_registers():
     (4 heads per wave: 168 of them) a wave per SIMD, 2 workgroups of 4 waves per CU for 3."""
     cus = torch.cuda.get_device_properties(DEV).multi_processor_count
     assert pa.decode_workgroups(DEV, torch.float32, 64, 16, 4) == 3 * cus
+
+
+def test_a_step_larger_than_q_is_refused():
+    """A mixed step's row indices reach past a q (or out) of fewer rows: an IndexError, as from
+    q[rows], and before any kernel that would skip such rows."""
+    cache = PagedKVCache(KVShape(1, 2, 64), 8, 16, "cpu", torch.bfloat16)
+    batch = PagedBatch.build(cache, [[0], [1, 2], [3]], [5, 20, 9], [1, 20, 9], "cpu", use_kernel=True)
+    assert batch.num_tokens == 30
+    q = torch.zeros(30, 4, 64, dtype=torch.bfloat16)
+    with pytest.raises(IndexError, match="30 tokens"):
+        mixed_attention(0, q[:29], batch)
+    with pytest.raises(IndexError, match="30 tokens"):
+        mixed_attention(0, q, batch, out=q[:29].clone())
