@@ -34,9 +34,10 @@ struct CascadeLaunch {
   int wslots, tail_slots;
 };
 
-// decode.hip: pkv_paged_decode_ex (rows, num_rows: pkv_paged_decode_rows); with `one`, the stream pass runs in one launch with
-// the prefix pass `one` describes (PKV_E_SHAPE where cascade_prefix_wg gives 0). With
-// check_only, every argument check runs and nothing is launched.
+// decode.hip: pkv_paged_decode_ex (rows, num_rows: pkv_paged_decode_rows); with `one`, the
+// stream pass runs in one launch with the prefix pass `one` describes (PKV_E_SHAPE where
+// cascade_prefix_wg gives 0). With check_only, every argument check runs and nothing is
+// launched.
 int decode_ex(void* out, int out_dtype, int64_t out_stride_b, int64_t out_stride_h,
               const void* q, int64_t q_stride_b, int64_t q_stride_h, const void* k_cache,
               const void* v_cache, int kv_dtype, int64_t kv_stride_slot, int64_t kv_stride_head,

@@ -361,11 +361,12 @@ std::mutex g_scratch_mu;
 // Whether a default-split call (num_workgroups == 0) takes the per-sequence split pass,
 // and with how many query heads per wave (*gpw, 0 = no): 16-bit K/V at head_dim 64 or
 // 128, no cascade extras, the table width bounds every wave's share to kSplitMaxTiles
-// tiles, and the (sequence, KV head, head sub-group) workgroups fit the CUs. The split
-// pass is bound by each wave's VALU work (its P.V runs per query head), so the fewest
-// heads per wave whose workgroups still fit the CUs is taken: more CUs at work, each
-// wave's K/V re-read by the head sub-groups from cache. Static shapes only, so a
-// captured graph stays valid for every context length.
+// tiles, and the (sequence, KV head, head sub-group) workgroups fit the CUs. Up to 4 heads
+// per wave the split pass is bound by each wave's VALU work (P.V per query head), so the
+// fewest heads whose workgroups still fit the CUs are taken: more CUs at work, each wave's
+// K/V re-read by the head sub-groups from cache. Past 4 heads a wave is of the wide form,
+// whose P.V runs on the matrix cores. Static shapes only, so a captured graph stays valid
+// for every context length.
 int choose_split(int kv_dtype, int head_dim, int batch, int num_heads, int num_kv_heads,
                  int max_columns, int64_t max_tokens, bool extras, int* gpw) {
   *gpw = 0;

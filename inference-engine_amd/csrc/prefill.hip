@@ -34,7 +34,9 @@ using namespace pkv;
 // before (16 tokens per workgroup, scores and P.V on the VALU, no load in flight under the
 // arithmetic) and now, fp32: 8 x 300 tokens behind up to 1,500, 32 / 8 heads, hd 128: 3,154 ->
 // 547; 3 x 100-300 behind up to 700, hd 128: 371 -> 83; 1,000 tokens, hd 64: 234 -> 62; 20
-// behind 2,000: 54 -> 17; 2 x 100-300, hd 256: 144 -> 68; bf16 at hd 16, 4 x 100-400: 93 -> 16.
+// behind 2,000: 54 -> 17; 2 x 100-300, hd 256: 144 -> 68; bf16 at hd 16, 4 x 100-400: 93 -> 16;
+// with one query head per KV head, where 64 rows are 64 tokens: 64 tokens, 4 heads, hd 64 9.2 ->
+// 8.9, 32 heads, hd 128 13.4 -> 12.5; 256 chunks of 4, 4 heads, hd 64 55 -> 42.
 // Error against 64 bits on 3 chunks of 60-300 tokens, hd 64: 3.5e-7 -> 3.2e-7.
 // ---------------------------------------------------------------------------------
 

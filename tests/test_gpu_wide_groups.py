@@ -30,8 +30,8 @@ def _exact(step):
 
 
 def _tol(step):
-    """|V| < 6 times P's relative error -- 2^-22 at hd 128 (three bf16 or two fp16 terms), 2^-17
-    at hd 64 (two bf16 terms) -- plus fp32 scores of a few ulps (|s| < 16) and fp32 sums."""
+    """|V| < 6 times P's relative error -- 2^-22 holds it at hd 128 (fp32, or three bf16 terms) and
+    for two fp16 terms at hd 64, 2^-17 two bf16 terms at hd 64 -- plus fp32 scores of a few ulps (|s| < 16) and fp32 sums."""
     p = 2.0**-17 if step.q.shape[-1] == 64 and step.q.dtype == torch.bfloat16 else 2.0**-22
     return 6 * (p + 16 * 2.0**-23)
 
