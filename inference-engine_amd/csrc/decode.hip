@@ -112,8 +112,10 @@ template <int DT, int HD, int GPW> constexpr unsigned stream_lds(int wpg) {
 //   1,024 pairs (32 of 2,060-2,200)                 56.9 / 54.5 / 56.1 / 57.2 / 64.4
 //   32 pairs, hd 256 (1 of 20,011)                  65.6 / 54.0 / 47.0 / 44.4 / 44.4
 //   8 pairs, hd 256 (1 of 9,000, 8 heads)          122.2 / 74.6 / 43.8 / 34.0 / 30.3
-// (Four waves up to 1,024 pairs gain 0.5-1% where a few long sequences have most of the ranges, 32
-// of 128-32,768, and lose 1-3% elsewhere.)
+// (Two libraries in turn on the same buffers, hd 128: four waves up to 1,024 pairs gain 0.4-0.9%
+// where a few long sequences have most of the ranges, 32 or 24 of 128-32,768, and lose 1-2% where
+// lengths are even: 45.3 against 45.9 us for 64 of 200-3,000, 55.9 against 56.6 for 32 of
+// 2,060-2,200.)
 int combine_waves(const DecodeArgs& a) {
   const int pairs = a.batch * a.nh;
   if (pairs <= 64) return 16;
