@@ -307,12 +307,11 @@ int32_t plan_workgroups(const DecodePlan& p, int kv_dtype, int head_dim) {
 // Ranges of the default stream-K split of a batch whose tables hold `max_tokens` tokens: what the
 // device holds at once, but for the wide form, whose ranges cost more (a record of up to 16 heads
 // for each, folded by the combine). There (us per call at this many ranges):
-//   * four waves per CU where the ranges would hold fewer than 24 tiles of 16 tokens: 16 / 1
-//     heads, 64 sequences of 100-3,943 tokens, 2,048 / 1,024 ranges 30.1 / 27.6; 32 / 2, 1,024 /
-//     512 39.8 / 37.4; but 130 of 100-3,841, fp16 (30 tiles), 63.0 / 74.6;
-//   * past one workgroup per CU, at least gpw / 2 tiles per range: its records are then a quarter
-//     of the K/V it reads (64 / 4, one sequence of 20,011 tokens, 512 / 256 ranges 31.4 / 23.5;
-//     8 / 1, 300 of 20-99, 2,048 / 1,024 / 512 20.7 / 16.5 / 15.9);
+//   * past one workgroup per CU, at least gpw / 2 tiles of 16 tokens per range: its records are
+//     then a quarter of the K/V it reads (64 / 4, one sequence of 20,011 tokens, 512 / 256 ranges
+//     31.4 / 23.5; 8 / 1, 300 of 20-99, 2,048 / 1,024 / 512 20.7 / 16.5 / 15.9). Fewer for longer
+//     ranges too gain in bf16 (32 / 2, 64 of 100-3,943, 15 tiles in each of 1,024 39.8, 512 37.4)
+//     and lose in fp16, whose matrix work is longer (16 / 2, the same 38.8, 44.5);
 //   * up to there, at least gpw / 4, down to 64 ranges: 128 / 8, one sequence of 2,500, 256 / 128
 //     / 64 21.7 / 18.6 / 17.5 (18.2 in waves of 4 heads); of 8,000, 256 / 128 / 64 27.1 / 24.2 /
 //     27.2; 64 / 8, of 8,000, 256 / 128 21.6 / 20.7.
@@ -324,7 +323,6 @@ int32_t default_ranges(const DecodePlan& p, int kv_dtype, int head_dim, int batc
   if (st) return st;
   const int64_t tiles = (int64_t)batch * ((max_tokens + 15) / 16);
   int64_t r = full;
-  if (tiles < 24 * r) r = std::min<int64_t>(r, (int64_t)cus * ((p.wpg + 3) / p.wpg));
   if (r > cus) r = std::max<int64_t>(cus, std::min(r, tiles * 2 / p.gpw / cus * cus));
   if (r <= cus) r = std::max(std::min<int64_t>(r, 64), std::min(r, (tiles * 4 / p.gpw + 7) / 8 * 8));
   return (int32_t)r;

@@ -1341,9 +1341,8 @@ __device__ __forceinline__ void decode_mfma_body(const DecodeArgs& a, const int 
     if constexpr (kTerms) {
       bool nan = false;
 #pragma unroll
-      for (int d = 0; d < NOV; ++d)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) nan = nan || ov[d][r] != ov[d][r];
+      for (int d = 0; d < NOV; ++d)  // two values per comparison
+        nan = nan || __builtin_isunordered(ov[d][0], ov[d][1]) || __builtin_isunordered(ov[d][2], ov[d][3]);
       v_careful = __builtin_amdgcn_ballot_w64(nan && col < ng) != 0;
       if (!v_careful) break;
     }
